@@ -71,7 +71,7 @@ DeviceTables g_dev[kMaxDevices];
 Registry<float>* g_rf = nullptr;
 Registry<double>* g_rd = nullptr;
 int g_sel[2][3][kLogMax + 1];  // [dtype][kind: rows, cols, chain][log2 n] -> variant
-int g_chunk[2][kLogMax + 1];   // fields per three-sweep chunk (0 = whole batch)
+int g_chunk[2][kLogMax + 1];   // fields per three-sweep chunk (0 = chunk_fields' choice)
 
 // A plan's copy of the selection for its (dtype, log2 n), taken at lp2d_plan_create;
 // during a plan call it is the calling thread's selection for that size, so later
@@ -354,16 +354,18 @@ int run_small(const PassArgs<T>& a, int lg, int mode, hipStream_t s) {
 // measured 1.6x slower, more than the tiled column pass gains.)
 template <typename T>
 const RowVar<T>& grad_variant(int lg) {
-  int vi = 0;
-  for (int i = 1; i < reg<T>()->nrows[lg]; ++i)
-    if (reg<T>()->rows[lg][i].E < reg<T>()->rows[lg][vi].E) vi = i;
+  int vi = -1;
+  for (int i = 0; i < reg<T>()->nrows[lg]; ++i) {
+    const RowVar<T>& v = reg<T>()->rows[lg][i];
+    if (v.grad_fn && (vi < 0 || v.E < reg<T>()->rows[lg][vi].E)) vi = i;
+  }
   return reg<T>()->rows[lg][vi];
 }
 
 // F_TILED when the selected schedules can hand the intermediate plane between the
-// sweeps over in the block-tiled layout: the pipelined complex64 column class with
-// strips of tile_cols(n), row tiles of whole tile_rows(n)-row blocks, and (grad) the
-// adjoint's gradient pass reading it (whole blocks again, unless it stores nothing).
+// sweeps over in the block-tiled layout: the complex64 column strips by occupancy, row
+// tiles of whole tile_rows(n)-row blocks, and (grad) the adjoint's gradient pass reading
+// it (whole blocks again, unless it stores nothing).
 template <typename T>
 int tiled_flag(const PassArgs<T>& cols_a, int lg, bool grad = false, bool grad_store = true) {
   if (sizeof(T) != 4) return 0;
@@ -371,8 +373,9 @@ int tiled_flag(const PassArgs<T>& cols_a, int lg, bool grad = false, bool grad_s
   const ColVar<T>& cv = reg<T>()->cols[lg][sel_of(dt<T>(), 1, lg)];
   const RowVar<T>& rv = reg<T>()->rows[lg][sel_of(dt<T>(), 0, lg)];
   const int tr = tile_rows(n), tc = tile_cols(n);
-  if (!(cv.kind & 2) || cv.W != tc || (n / cv.E) % tr != 0) return 0;
-  if (!pipe_eligible(cols_a, MODE_FWD | MODE_INV)) return 0;
+  if (!(cv.kind & 8) || (n / cv.E) % tr != 0) return 0;
+  if (cv.W % tc != 0 && tc % cv.W != 0) return 0;
+  if (!occ_eligible(cols_a, MODE_FWD | MODE_INV)) return 0;
   if (rv.lines % tr != 0 || (n / rv.E) % tc != 0) return 0;
   if (grad) {
     const RowVar<T>& gv = grad_variant<T>(lg);
@@ -673,14 +676,30 @@ template <typename T>
 int op_propagate_chunk(int n, int lg, int batch, const void* in, void* out, const float* phase,
                        int64_t phase_sb, const lp2d_optics* o, void* spec, hipStream_t s);
 
-// Field-to-field propagation.  Large sizes run three sweeps per chunk of fields so
-// that a chunk's intermediate planes are still in the Infinity Cache when the next
-// sweep reads them (chunk size from lp2d_set_chunk; 0 = the whole batch at once).
+// Fields of one three-sweep call that run together: lp2d_set_chunk's choice, or as many
+// as keep their intermediate planes within the 256 MB Infinity Cache between the sweeps
+// (a copy in place runs at 8.4 TB/s up to there and 5.6 TB/s from memory).  Measured,
+// complex64, whole batch against chunks of 256 MB: 2048 x 256^2 1146 -> 953 us, 512 x
+// 512^2 1165 -> 1004, 128 x 1024^2 1203 -> 1049, 4 x 4096^2 779 -> 693, 5 x 4096^2 1167 ->
+// 924; complex128 8 x 2048^2 635 -> 572.  Half that size costs 7-10 % more (the fixed
+// cost of a launch).  A single field larger than that cannot be split.
+constexpr long long kChunkBytes = 256LL << 20;
+template <typename T>
+int chunk_fields(int lg, int batch) {
+  const int set = chunk_of(dt<T>(), lg);
+  if (set > 0) return set < batch ? set : batch;
+  const long long field = (long long)sizeof(cx<T>) << (2 * lg);
+  if (field > kChunkBytes || field * batch <= kChunkBytes) return batch;
+  return (int)(kChunkBytes / field);
+}
+
+// Field-to-field propagation, three sweeps per chunk of fields.
 template <typename T>
 int op_propagate(int n, int lg, int batch, const void* in, void* out, const float* phase,
                  int64_t phase_sb, const lp2d_optics* o, void* spec, hipStream_t s) {
-  const int chunk = chunk_of(dt<T>(), lg);
-  if (chunk <= 0 || chunk >= batch || use_small<T>(lg))
+  ensure_registry();
+  const int chunk = use_small<T>(lg) ? batch : chunk_fields<T>(lg, batch);
+  if (chunk >= batch)
     return op_propagate_chunk<T>(n, lg, batch, in, out, phase, phase_sb, o, spec, s);
   const long long fs = (long long)n * n;
   for (int c0 = 0; c0 < batch; c0 += chunk) {
@@ -760,11 +779,17 @@ int grad_groups(int lg, int batch) {
 //   -> cols -> inverse rows,
 // 2K + 1 sweeps instead of 3K, in the output buffer; the chain passes store the plane
 // inputs u_k that planes[k] asks for.  Otherwise one fused propagation per plane.
+// Fields [b0, b0 + batch) of the call; op_stack runs it chunk by chunk.
 template <typename T>
-int op_stack(int n, int lg, int batch, const void* in, void* out, const float* screens, int K,
-             const lp2d_optics* o, void* const* planes, hipStream_t s) {
+int op_stack_chunk(int n, int lg, int b0, int batch, const void* in, void* out,
+                   const float* screens, int K, const lp2d_optics* o, void* const* planes,
+                   hipStream_t s) {
   const long long nn = (long long)n * n;
-  auto plane = [&](int k) -> void* { return (planes && k > 0 && k < K) ? planes[k] : nullptr; };
+  in = (const cx<T>*)in + b0 * nn;
+  out = (cx<T>*)out + b0 * nn;
+  auto plane = [&](int k) -> void* {
+    return (planes && k > 0 && k < K && planes[k]) ? (cx<T>*)planes[k] + b0 * nn : nullptr;
+  };
   DeviceTables* t;
   if (int rc = current_tables(&t, s)) return rc;
   PassArgs<T> a = base_args<T>(t, n, batch);
@@ -825,6 +850,21 @@ int op_stack(int n, int lg, int batch, const void* in, void* out, const float* s
       e = chain(r, s);
     }
     if (e != hipSuccess) return hip_fail(e, "chained row pass launch");
+  }
+  return LP2D_OK;
+}
+
+template <typename T>
+int op_stack(int n, int lg, int batch, const void* in, void* out, const float* screens, int K,
+             const lp2d_optics* o, void* const* planes, hipStream_t s) {
+  // (the chained sweeps gain from chunks up to 1024 points, 5 screens: 2048 x 256^2 4457
+  // -> 3806 us, 128 x 1024^2 5009 -> 4794; 16 x 2048^2 3493 -> 3641, 8 x 4096^2 6.4 -> 6.9
+  // ms)
+  const bool whole = use_small<T>(lg) || (lg > 10 && chunk_of(dt<T>(), lg) == 0);
+  const int chunk = whole ? batch : chunk_fields<T>(lg, batch);
+  for (int c0 = 0; c0 < batch; c0 += chunk) {
+    const int cb = batch - c0 < chunk ? batch - c0 : chunk;
+    if (int rc = op_stack_chunk<T>(n, lg, c0, cb, in, out, screens, K, o, planes, s)) return rc;
   }
   return LP2D_OK;
 }
@@ -1056,14 +1096,22 @@ int run_bucket(const Bucket& bk, hipStream_t s) {
   }
   a.flags = bk.flags;
   const int tl = tiled_flag<T>(a, bk.lg);
-  a.flags = tl;
-  if (int rc = run_rows<T>(a, bk.lg, false, s)) return rc;
-  a.src_tab = (const cx<T>* const*)bk.d_dst;  // later sweeps work in the destinations
-  a.flags = bk.flags | tl;
-  if (int rc = run_cols<T>(a, bk.lg, MODE_FWD | MODE_INV, s)) return rc;
-  a.flags = F_SCALE | tl;
-  a.scale = sc;
-  return run_rows<T>(a, bk.lg, true, s);
+  const int chunk = chunk_fields<T>(bk.lg, bk.count);
+  for (int c0 = 0; c0 < bk.count; c0 += chunk) {
+    a.batch = bk.count - c0 < chunk ? bk.count - c0 : chunk;
+    a.fopt = bk.d_opt + c0;
+    a.src_tab = (const cx<T>* const*)bk.d_src + c0;
+    a.dst_tab = (cx<T>* const*)bk.d_dst + c0;
+    a.flags = tl;
+    if (int rc = run_rows<T>(a, bk.lg, false, s)) return rc;
+    a.src_tab = (const cx<T>* const*)bk.d_dst + c0;  // later sweeps work in the destinations
+    a.flags = bk.flags | tl;
+    if (int rc = run_cols<T>(a, bk.lg, MODE_FWD | MODE_INV, s)) return rc;
+    a.flags = F_SCALE | tl;
+    a.scale = sc;
+    if (int rc = run_rows<T>(a, bk.lg, true, s)) return rc;
+  }
+  return LP2D_OK;
 }
 
 }  // namespace
@@ -1673,7 +1721,7 @@ int lp2d_variant_name(int n, int dtype, int kind, int variant, char* buf, int bu
     const int lds = dtype ? g_rd->rows[lg][variant].lds : g_rf->rows[lg][variant].lds;
     const int rk = dtype ? g_rd->rows[lg][variant].kind : g_rf->rows[lg][variant].kind;
     return snprintf(buf, buflen, "rows E=%d lines=%d threads=%d lds=%d%s", E, L, th, lds,
-                    (rk & 2) ? " pipelined" : (rk & 4) ? " lds-twiddles" : "");
+                    (rk & 8) ? " one-tile" : "");
   }
   const int E = dtype ? g_rd->cols[lg][variant].E : g_rf->cols[lg][variant].E;
   const int W = dtype ? g_rd->cols[lg][variant].W : g_rf->cols[lg][variant].W;
@@ -1681,7 +1729,7 @@ int lp2d_variant_name(int n, int dtype, int kind, int variant, char* buf, int bu
   const int lds = dtype ? g_rd->cols[lg][variant].lds : g_rf->cols[lg][variant].lds;
   const int ck = dtype ? g_rd->cols[lg][variant].kind : g_rf->cols[lg][variant].kind;
   return snprintf(buf, buflen, "cols E=%d W=%d threads=%d lds=%d%s%s", E, W, th, lds,
-                  (ck & 2) ? " pipelined" : "", (ck & 1) ? " shared-H" : "");
+                  (ck & 8) ? " one-strip" : "", (ck & 1) ? " shared-H" : "");
 }
 
 }  // extern "C"

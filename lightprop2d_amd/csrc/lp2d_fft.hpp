@@ -288,24 +288,32 @@ __device__ __forceinline__ void line_fft(cx<T> (&v)[E], int t, const Acc& acc,
 // up to 16, whose w^{rk} come from the product tree w^{rk} = w^{(r-r/2)k} w^{(r/2)k}
 // (at most 1 + log2(r) roundings); so that 2-row tiles of 4096 points and their
 // tables fit twice in one CU's LDS.
+// CL = 3 (split compact last pass, one pair of tables per r): w^{rk} = w^{r*S*(k/S)} *
+// w^{r*(k%S)}, each factor read from a table of rows like the full one's (S + NS/S rows:
+// 2.5 KB for n = 2048 with 16 elements per thread).  Every twiddle is one product of two
+// table entries, where the product tree multiplies the error of w^k by r: n = 2048,
+// whole propagation against 64 bits 4.3e-7 with the tree, 3.0e-7 with the full table.
+// CL = 4 (half compact, a last pass of radix 2): w^k for k < NS/2, the other half being
+// w^k = -i * w^{k - NS/2} exactly.
 constexpr int twl_radix(int N, int E, int ns) { return N / ns >= E ? E : N / ns; }
 constexpr bool twl_compact(int N, int E, int ns, int CL) {
   return CL != 0 && ns > 1 && ns * twl_radix(N, E, ns) == N &&
-         twl_radix(N, E, ns) <= (CL == 2 ? 16 : 4);
+         twl_radix(N, E, ns) <= (CL >= 2 ? 16 : 4);
 }
 constexpr int twl_split(int ns) {
   int l = 0;
   while ((2 << l) <= ns) ++l;
   return 1 << (l / 2);
 }
-constexpr int twl_compact_len(int ns, int CL) {
-  return CL == 2 ? twl_split(ns) + ns / twl_split(ns) : ns;
+constexpr int twl_compact_len(int ns, int R, int CL) {
+  if (CL == 4) return ns / 2;
+  return CL >= 2 ? (twl_split(ns) + ns / twl_split(ns)) * (CL == 3 ? R + 2 : 1) : ns;
 }
 constexpr int twl_off(int N, int E, int NS, int CL = 0) {
   int off = 0;
   for (int ns = 1; ns < NS; ns *= twl_radix(N, E, ns))
     if (ns > 1)
-      off += twl_compact(N, E, ns, CL) ? twl_compact_len(ns, CL)
+      off += twl_compact(N, E, ns, CL) ? twl_compact_len(ns, twl_radix(N, E, ns), CL)
                                        : ns * (twl_radix(N, E, ns) + 2);
   return off;
 }
@@ -315,24 +323,58 @@ struct TwlLen {
 };
 
 // Fill the per-pass tables from the concatenated global table (size L at offset L-2).
+// All of a thread's loads are issued before its first LDS write, so a short-lived
+// workgroup waits for one round trip and not for one per entry.
+template <typename T, int LEN, int THREADS, typename Src, typename Dst>
+__device__ __forceinline__ void twl_copy(cx<T>* twl, const cx<T>* __restrict__ tw, int tid,
+                                         Src&& src, Dst&& dst) {
+  constexpr int CNT = (LEN + THREADS - 1) / THREADS;
+  cx<T> v[CNT];
+#pragma unroll
+  for (int c = 0; c < CNT; ++c) {
+    const int i = tid + c * THREADS;
+    if (LEN % THREADS == 0 || i < LEN) v[c] = tw[src(i)];
+  }
+#pragma unroll
+  for (int c = 0; c < CNT; ++c) {
+    const int i = tid + c * THREADS;
+    if (LEN % THREADS == 0 || i < LEN) twl[dst(i)] = v[c];
+  }
+}
 template <typename T, int N, int E, int THREADS, int NS = 1, int CL = 0>
 __device__ __forceinline__ void twl_fill(cx<T>* twl, const cx<T>* __restrict__ tw, int tid) {
   if constexpr (NS < N) {
     constexpr int R = twl_radix(N, E, NS);
+    constexpr int L = NS * R, OFF = twl_off(N, E, NS, CL);
     if constexpr (twl_compact(N, E, NS, CL) && CL == 2) {
       // w^i for i < S, then w^{S*h} for h < NS/S
-      constexpr int L = NS * R, OFF = twl_off(N, E, NS, CL), S = twl_split(NS);
-      for (int i = tid; i < S + NS / S; i += THREADS)
-        twl[OFF + i] = tw[(L - 2) + (i < S ? i : (i - S) * S)];
+      constexpr int S = twl_split(NS);
+      twl_copy<T, S + NS / S, THREADS>(
+          twl, tw, tid, [](int i) { return (L - 2) + (i < S ? i : (i - S) * S); },
+          [](int i) { return OFF + i; });
+    } else if constexpr (twl_compact(N, E, NS, CL) && CL == 4) {
+      static_assert(R == 2, "half table");
+      twl_copy<T, NS / 2, THREADS>(
+          twl, tw, tid, [](int i) { return (L - 2) + i; }, [](int i) { return OFF + i; });
+    } else if constexpr (twl_compact(N, E, NS, CL) && CL == 3) {
+      // rows w^{r*i}, i < S, then w^{r*S*h}, h < NS/S (r < R; an entry is in the table:
+      // r*S*h < L)
+      constexpr int S = twl_split(NS), P = R + 2;
+      twl_copy<T, (S + NS / S) * R, THREADS>(
+          twl, tw, tid,
+          [](int i) {
+            const int q = i / R, r = i % R;
+            return (L - 2) + r * (q < S ? q : (q - S) * S);
+          },
+          [](int i) { return OFF + (i / R) * P + i % R; });
     } else if constexpr (twl_compact(N, E, NS, CL)) {
-      constexpr int L = NS * R, OFF = twl_off(N, E, NS, CL);
-      for (int i = tid; i < NS; i += THREADS) twl[OFF + i] = tw[(L - 2) + i];
+      twl_copy<T, NS, THREADS>(
+          twl, tw, tid, [](int i) { return (L - 2) + i; }, [](int i) { return OFF + i; });
     } else if constexpr (NS > 1) {
-      constexpr int L = NS * R, P = R + 2, OFF = twl_off(N, E, NS, CL);
-      for (int i = tid; i < L; i += THREADS) {
-        const int k = i / R, r = i % R;
-        twl[OFF + k * P + r] = tw[(L - 2) + k * r];
-      }
+      constexpr int P = R + 2;
+      twl_copy<T, L, THREADS>(
+          twl, tw, tid, [](int i) { return (L - 2) + (i / R) * (i % R); },
+          [](int i) { return OFF + (i / R) * P + i % R; });
     }
     twl_fill<T, N, E, THREADS, NS * R, CL>(twl, tw, tid);
   }
@@ -356,7 +398,21 @@ __device__ __forceinline__ void stockham_l(cx<T> (&v)[E], int t, const Acc& acc,
     cx<T> a[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) a[r] = v[q + r * B];
-    if constexpr (twl_compact(N, E, NS, CL)) {
+    if constexpr (twl_compact(N, E, NS, CL) && CL == 4) {
+      const cx<T> q = twl[twl_off(N, E, NS, CL) + (k & (NS / 2 - 1))];
+      const bool rot = k >= NS / 2;
+      const cx<T> w = mk(rot ? q.im : q.re, rot ? -q.re : q.im);
+      a[1] = INV ? cmulc(a[1], w) : cmul(a[1], w);
+    } else if constexpr (twl_compact(N, E, NS, CL) && CL == 3) {
+      constexpr int S = twl_split(NS), OFF = twl_off(N, E, NS, CL), P = R + 2;
+      const cx<T>* ta = twl + (OFF + (k & (S - 1)) * P);
+      const cx<T>* tb = twl + (OFF + (S + k / S) * P);
+#pragma unroll
+      for (int r = 1; r < R; ++r) {
+        const cx<T> w = cmul(tb[r], ta[r]);
+        a[r] = INV ? cmulc(a[r], w) : cmul(a[r], w);
+      }
+    } else if constexpr (twl_compact(N, E, NS, CL)) {
       // w^k from the table; w^{2k}, w^{3k} by products (R <= 4)
       cx<T> w[R > 1 ? R : 2];
       if constexpr (CL == 2) {

@@ -29,34 +29,22 @@ __global__ __launch_bounds__((N / E) * LINES) LP2D_OCC void k_rows(PassArgs<T> a
   rows_body<T, N, E, LINES, INV, PS, FEAT>(a, b, y0, cmin(LINES, N - y0), lds, threadIdx.x);
 }
 
-// The row pass with its twiddles staged once in LDS (compact mode CL), each workgroup
-// taking every gridDim.x-th row tile of the batch (one resident round).
-template <typename T, int N, int E, int LINES, bool INV, int PS, bool FEAT, int CL,
-          bool PHO = false>
-__global__ __launch_bounds__((N / E) * LINES) LP2D_OCC void k_rows_l(PassArgs<T> a, int nunits) {
+// The row pass of one tile per workgroup with its twiddles staged in LDS and each row's
+// threads in one wave.
+template <typename T, int N, int E, int LINES, bool INV, int PS, bool FEAT, int CL, bool PHO,
+          int WPE>
+__global__ __launch_bounds__((N / E) * LINES) __attribute__((amdgpu_waves_per_eu(WPE)))
+void k_rows_occ(PassArgs<T> a) {
   __shared__ cx<T> lds[LINES * RowPitch<N, PS, LINES>::value];
   __shared__ cx<T> twl[TwlLen<N, E, CL>::value];
+  static_assert(N % LINES == 0, "whole tiles");
+  constexpr int TPF = N / LINES;
   twl_fill<T, N, E, (N / E) * LINES, 1, CL>(twl, a.tw, threadIdx.x);
   __syncthreads();
-  constexpr int TPF = N / LINES;
-  for (int u = blockIdx.x; u < nunits; u += gridDim.x) {
-    const int b = u / TPF;
-    rows_body<T, N, E, LINES, INV, PS, FEAT, CL, PHO>(a, b, (u - b * TPF) * LINES, LINES, lds,
-                                                      threadIdx.x, twl);
-  }
-}
-
-// Pipelined row pass: about one resident round of workgroups, each taking every
-// gridDim.x-th row tile of the batch; the twiddle tables are staged in LDS once.
-template <typename T, int N, int E, int LINES, bool INV, int PS, bool TILED, bool PH = false,
-          bool WSK = true>
-__global__ __launch_bounds__((N / E) * LINES) LP2D_OCC void k_rows_pipe(PassArgs<T> a, int nunits) {
-  __shared__ cx<T> lds[LINES * RowPitch<N, PS, LINES>::value];
-  __shared__ cx<T> twl[TwlLen<N, E>::value];
-  twl_fill<T, N, E, (N / E) * LINES>(twl, a.tw, threadIdx.x);
-  __syncthreads();
-  rows_pipe_body<T, N, E, LINES, INV, PS, TILED, PH, WSK>(a, blockIdx.x, gridDim.x, nunits, lds,
-                                                          twl, threadIdx.x);
+  const int tile = blockIdx.x;
+  const int b = tile / TPF;
+  rows_occ_body<T, N, E, LINES, INV, PS, FEAT, CL, PHO>(a, b, (tile - b * TPF) * LINES, lds, twl,
+                                                        threadIdx.x);
 }
 
 // The pipelined gradient body when its screen factor is hoisted and the LDS twiddle
@@ -120,43 +108,34 @@ void k_rows_chain_l(PassArgs<T> a, int nunits) {
   }
 }
 
-// Grid: (N/W strips) x (field groups of `per` fields).
+// Grid: (N/W strips) x fields.
 template <typename T, int N, int E, int W, int MODE, int PS, int MIDK>
-__global__ __launch_bounds__((N / E) * W) LP2D_OCC void k_cols(PassArgs<T> a, int per) {
+__global__ __launch_bounds__((N / E) * W) LP2D_OCC void k_cols(PassArgs<T> a) {
   __shared__ cx<T> lds[W * PaddedLen<N, PS>::value];
   constexpr int SPF = N / W;  // column strips per field
   const int g = gridDim.x, i = blockIdx.x;
   // Workgroups go to the 8 XCDs round robin.  Give each XCD a contiguous run of
   // strips so that narrow strips sharing 128-byte lines meet in the same L2.
   const int blk = (g % 8 == 0) ? (i % 8) * (g / 8) + i / 8 : i;
-  const int grp = blk / SPF;
-  const int x0 = (blk - grp * SPF) * W;
-  const int b0 = grp * per;
-  const int b1 = cmin(a.batch, b0 + per);
-  cols_body<T, N, E, W, MODE, PS, MIDK>(a, b0, b1, x0, lds, threadIdx.x);
+  const int b = blk / SPF;
+  cols_body<T, N, E, W, MODE, PS, MIDK>(a, b, (blk - b * SPF) * W, lds, threadIdx.x);
 }
 
-// Pipelined column pass: grid (N/W strips) x (field groups of `per` <= kPipeMaxPer
-// fields); the twiddle tables of the strip's passes and the group's field pointers
-// and optics are staged in LDS once per workgroup.
-template <typename T, int N, int E, int W, int PS, int HOISTH = HOIST_NONE, int CL = 0>
-__global__ __launch_bounds__((N / E) * W) LP2D_OCC void k_cols_pipe(PassArgs<T> a, int per) {
+// Column strips by occupancy: grid (N/W strips) x (field groups of `per` fields).
+template <typename T, int N, int E, int W, int PS, int CL, bool SPEC, int WPE>
+__global__ __launch_bounds__((N / E) * W) __attribute__((amdgpu_waves_per_eu(WPE)))
+void k_cols_occ(PassArgs<T> a, int per) {
   __shared__ cx<T> lds[W * PaddedLen<N, PS>::value];
   __shared__ cx<T> twl[TwlLen<N, E, CL>::value];
-  __shared__ PipeField pf[kPipeMaxPer];
-  constexpr int THREADS = (N / E) * W;
-  static_assert(THREADS >= kPipeMaxPer, "one thread per staged field");
   constexpr int SPF = N / W;
   const int g = gridDim.x, i = blockIdx.x;
   const int blk = (g % 8 == 0) ? (i % 8) * (g / 8) + i / 8 : i;
   const int grp = blk / SPF;
-  const int x0 = (blk - grp * SPF) * W;
   const int b0 = grp * per;
-  const int b1 = cmin(a.batch, b0 + per);
-  twl_fill<T, N, E, THREADS, 1, CL>(twl, a.tw, threadIdx.x);
-  pipe_stage_fields(a, b0, b1, pf, threadIdx.x);
+  twl_fill<T, N, E, (N / E) * W, 1, CL>(twl, a.tw, threadIdx.x);
   __syncthreads();
-  cols_pipe_body<T, N, E, W, PS, HOISTH, CL>(a, b0, b1, x0, lds, twl, pf, threadIdx.x);
+  cols_occ_body<T, N, E, W, PS, CL, SPEC>(a, b0, cmin(a.batch, b0 + per), (blk - grp * SPF) * W,
+                                          lds, twl, threadIdx.x);
 }
 
 // Whole field in LDS, pipelined over groups of `per` <= kPipeMaxPer fields.
@@ -245,93 +224,27 @@ hipError_t launch_rows(const PassArgs<T>& a, bool inv, hipStream_t s) {
   return hipGetLastError();
 }
 
-template <typename T, int N, int E, int LINES, bool INV, int PS, bool FEAT, int CL, bool PHO>
-hipError_t run_rows_l(const PassArgs<T>& a, int nu, hipStream_t s) {
-  constexpr int threads = (N / E) * LINES;
-  static std::atomic<int> slot{0};
-  const int sl = cached_slots(
-      slot, (const void*)&k_rows_l<T, N, E, LINES, INV, PS, FEAT, CL, PHO>, threads);
-  const int grid = nu < sl ? nu : sl;
-  k_rows_l<T, N, E, LINES, INV, PS, FEAT, CL, PHO><<<grid, threads, 0, s>>>(a, nu);
-  return hipGetLastError();
-}
-template <typename T, int N, int E, int LINES, int PS, int CL>
-hipError_t launch_rows_l(const PassArgs<T>& a, bool inv, hipStream_t s) {
+// One tile per workgroup, rows within waves; every feature and the per-field tables.
+template <typename T, int N, int E, int LINES, int PS, int CL, int WPE>
+hipError_t launch_rows_occ(const PassArgs<T>& a, bool inv, hipStream_t s) {
   if ((a.flags & F_TILED) && (LINES % tile_rows(N) != 0 || (N / E) % tile_cols(N) != 0))
     return hipErrorInvalidValue;
-  // passes with spatial features keep the plain class (in the persistent loop their
-  // extra state spills: 636-748 bytes per lane at 4096 points), except a forward pass
-  // whose only feature is a phase screen
-  const long long units = (long long)a.batch * (N / LINES);
-  const int fl = a.flags & (F_SPATIAL | F_GRAD | F_INTENSITY | F_NO_STORE);
-  const bool pho = !inv && fl == F_PHASE && a.phase;
-  if ((fl != 0 && !pho) || N % LINES != 0 || units > 0x7fffffff)
-    return launch_rows<T, N, E, LINES, PS>(a, inv, s);
-  const int nu = (int)units;
-  if (pho) return run_rows_l<T, N, E, LINES, false, PS, false, CL, true>(a, nu, s);
-  return inv ? run_rows_l<T, N, E, LINES, true, PS, false, CL, false>(a, nu, s)
-             : run_rows_l<T, N, E, LINES, false, PS, false, CL, false>(a, nu, s);
-}
-
-// The pipelined class covers the row passes of strided complex64 batches without
-// spatial features (the passes of a plain propagation); anything else runs the plain
-// class of the same shape.  (Over an uneven batch's per-field pointer tables, read one
-// tile ahead, it measured slower than the plain class: 2.43 against 2.36 ms for
-// 2048 x 128^2 + 1536 x 256^2 + 512 x 512^2.)
-template <typename T, int N, int E, int LINES, bool INV, int PS, bool TILED, bool PH,
-          bool WSK = true>
-hipError_t run_rows_pipe_k(const PassArgs<T>& a, int nu, hipStream_t s) {
   constexpr int threads = (N / E) * LINES;
-  // same value on every thread that races to set it
-  static std::atomic<int> slot{0};
-  const int sl = cached_slots(
-      slot, (const void*)&k_rows_pipe<T, N, E, LINES, INV, PS, TILED, PH, WSK>, threads);
-  const int grid = nu < sl ? nu : sl;
-  k_rows_pipe<T, N, E, LINES, INV, PS, TILED, PH, WSK><<<grid, threads, 0, s>>>(a, nu);
+  const unsigned grid = (unsigned)((long long)a.batch * (N / LINES));
+  const int fl = a.flags & (F_SPATIAL | F_GRAD | F_INTENSITY | F_NO_STORE);
+  if (inv) {
+    if (fl)
+      k_rows_occ<T, N, E, LINES, true, PS, true, CL, false, 2><<<grid, threads, 0, s>>>(a);
+    else
+      k_rows_occ<T, N, E, LINES, true, PS, false, CL, false, WPE><<<grid, threads, 0, s>>>(a);
+  } else if (fl == F_PHASE && a.phase) {
+    k_rows_occ<T, N, E, LINES, false, PS, false, CL, true, WPE><<<grid, threads, 0, s>>>(a);
+  } else if (fl) {
+    k_rows_occ<T, N, E, LINES, false, PS, true, CL, false, 2><<<grid, threads, 0, s>>>(a);
+  } else {
+    k_rows_occ<T, N, E, LINES, false, PS, false, CL, false, WPE><<<grid, threads, 0, s>>>(a);
+  }
   return hipGetLastError();
-}
-// A pass converting between the natural and the block-tiled layout in place keeps the
-// workgroup-synchronised transform (the wave-local one would let a wave store over
-// data another wave has yet to load).
-template <typename T, int N, int E, int LINES, bool INV, int PS, bool TILED, bool PH>
-hipError_t run_rows_pipe(const PassArgs<T>& a, int nu, hipStream_t s) {
-  if constexpr (TILED) {
-    if ((const void*)a.src == (const void*)a.dst)
-      return run_rows_pipe_k<T, N, E, LINES, INV, PS, TILED, PH, false>(a, nu, s);
-  }
-  return run_rows_pipe_k<T, N, E, LINES, INV, PS, TILED, PH, true>(a, nu, s);
-}
-
-template <typename T, int N, int E, int LINES, int PS>
-hipError_t launch_rows_pipe(const PassArgs<T>& a, bool inv, hipStream_t s) {
-  constexpr bool TILE_OK = LINES % tile_rows(N) == 0 && (N / E) % tile_cols(N) == 0;
-  if ((a.flags & F_TILED) && !TILE_OK) return hipErrorInvalidValue;
-  if constexpr (sizeof(T) == 4 && N % LINES == 0) {
-    const int fl = a.flags & (F_SPATIAL | F_GRAD | F_INTENSITY | F_NO_STORE);
-    // the forward pass may carry a phase screen alone (shared or per field); at 512
-    // points its prefetched screen values spill (136 bytes per lane), and the plain
-    // pass with the screen prologue runs instead
-    constexpr bool PH_OK = N != 512;
-    const bool ph = PH_OK && !inv && fl == F_PHASE && a.phase;
-    const long long units = (long long)a.batch * (N / LINES);
-    if ((fl == 0 || ph) && !a.src_tab && !a.dst_tab && units <= 0x7fffffff) {
-      const bool tiled = (a.flags & F_TILED) != 0;
-      const int nu = (int)units;
-      if constexpr (TILE_OK) {
-        if (tiled) {
-          if (inv) return run_rows_pipe<T, N, E, LINES, true, PS, true, false>(a, nu, s);
-          if constexpr (PH_OK)
-            if (ph) return run_rows_pipe<T, N, E, LINES, false, PS, true, true>(a, nu, s);
-          return run_rows_pipe<T, N, E, LINES, false, PS, true, false>(a, nu, s);
-        }
-      }
-      if (inv) return run_rows_pipe<T, N, E, LINES, true, PS, false, false>(a, nu, s);
-      if constexpr (PH_OK)
-        if (ph) return run_rows_pipe<T, N, E, LINES, false, PS, false, true>(a, nu, s);
-      return run_rows_pipe<T, N, E, LINES, false, PS, false, false>(a, nu, s);
-    }
-  }
-  return launch_rows<T, N, E, LINES, PS>(a, inv, s);
 }
 
 template <typename T, int N, int E, int LINES, int PS, bool HOIST>
@@ -444,116 +357,91 @@ hipError_t launch_rows_adj_chain(const PassArgs<T>& a, int groups, float* partia
   }
 }
 
-// Fields per column workgroup: share the transfer function across a group of fields
-// while keeping at least ~kColBlocks workgroups in flight.
-constexpr int kColBlocks = 1024;
-
-template <typename T, int N, int E, int W, int PS, bool HOIST>
+template <typename T, int N, int E, int W, int PS>
 hipError_t launch_cols(const PassArgs<T>& a, int mode, hipStream_t s) {
   if (a.flags & F_TILED) return hipErrorInvalidValue;  // natural layout only
   constexpr int threads = (N / E) * W;
   constexpr int SPF = N / W;
-  // the shared-factor class needs one set of optics for the whole call
-  const bool hoist = HOIST && a.fopt == nullptr;
-  const bool shared_h = hoist && (a.flags & F_MID) && !(a.flags & (F_SMASK0 | F_SMASK1));
-  int per = shared_h ? (int)((long long)a.batch * SPF / kColBlocks) : 1;
-  if (per < 1) per = 1;
-  if (per > 8) per = 8;
-  const int groups = (a.batch + per - 1) / per;
-  const unsigned grid = (unsigned)((long long)groups * SPF);
+  const unsigned grid = (unsigned)((long long)a.batch * SPF);
   // spectral stage class: none / transfer function + aperture + store / with masks
   const int midk = (a.flags & (F_SMASK0 | F_SMASK1)) ? 2 : (a.flags & F_MID) ? 1 : 0;
   constexpr int FI = MODE_FWD | MODE_INV;
   switch (mode * 4 + midk) {
     case MODE_FWD * 4 + 0:
-      k_cols<T, N, E, W, MODE_FWD, PS, 0><<<grid, threads, 0, s>>>(a, per);
+      k_cols<T, N, E, W, MODE_FWD, PS, 0><<<grid, threads, 0, s>>>(a);
       break;
     case MODE_INV * 4 + 0:
-      k_cols<T, N, E, W, MODE_INV, PS, 0><<<grid, threads, 0, s>>>(a, per);
+      k_cols<T, N, E, W, MODE_INV, PS, 0><<<grid, threads, 0, s>>>(a);
       break;
     case MODE_INV * 4 + 1:
-      if constexpr (HOIST) {
-        if (hoist) {
-          k_cols<T, N, E, W, MODE_INV, PS, 3><<<grid, threads, 0, s>>>(a, per);
-          break;
-        }
-      }
-      k_cols<T, N, E, W, MODE_INV, PS, 1><<<grid, threads, 0, s>>>(a, per);
+      k_cols<T, N, E, W, MODE_INV, PS, 1><<<grid, threads, 0, s>>>(a);
       break;
     case FI * 4 + 0:
     case FI * 4 + 1:
-      if constexpr (HOIST) {
-        if (hoist) {
-          k_cols<T, N, E, W, FI, PS, 3><<<grid, threads, 0, s>>>(a, per);
-          break;
-        }
-      }
-      k_cols<T, N, E, W, FI, PS, 1><<<grid, threads, 0, s>>>(a, per);
+      k_cols<T, N, E, W, FI, PS, 1><<<grid, threads, 0, s>>>(a);
       break;
     case FI * 4 + 2:
-      k_cols<T, N, E, W, FI, PS, 2><<<grid, threads, 0, s>>>(a, per);
+      k_cols<T, N, E, W, FI, PS, 2><<<grid, threads, 0, s>>>(a);
       break;
     default:  // forward-only passes with a spectral stage, and inverse ones with masks
       if (mode == MODE_FWD)
-        k_cols<T, N, E, W, MODE_FWD, PS, 2><<<grid, threads, 0, s>>>(a, per);
+        k_cols<T, N, E, W, MODE_FWD, PS, 2><<<grid, threads, 0, s>>>(a);
       else
-        k_cols<T, N, E, W, MODE_INV, PS, 2><<<grid, threads, 0, s>>>(a, per);
+        k_cols<T, N, E, W, MODE_INV, PS, 2><<<grid, threads, 0, s>>>(a);
       break;
   }
   return hipGetLastError();
 }
 
-// The pipelined class covers the fused forward+inverse column pass of the complex64
-// path with transfer function / pupil / spectrum output; anything else (mask
-// multipliers, other evanescent modes, single-direction passes) runs the plain class
-// of the same shape.  Each workgroup takes `per` fields so that the grid is about one
-// round of resident workgroups.
-template <typename T, int N, int E, int W, int PS, int HOISTH = HOIST_NONE, int CL = 0>
-hipError_t launch_cols_pipe(const PassArgs<T>& a, int mode, hipStream_t s) {
-  const bool ok = pipe_eligible(a, mode);
-  // the block-tiled layout is only defined for strips of tile_cols(N) columns, and only
-  // this class reads it
-  if ((a.flags & F_TILED) && (!ok || W != tile_cols(N) || (N / E) % tile_rows(N) != 0))
-    return hipErrorInvalidValue;
+// Column strips by occupancy for the calls of occ_eligible; anything else runs the plain
+// class of the same shape.  Groups of up to GMAX fields share one transfer function where
+// the call has one set of optics, sized so that the grid is one resident round; per-field
+// tables run one field per workgroup.  (256 MB of fields, groups of one against GMAX:
+// 256 points 81 / 70 us, 512 84 / 78, 1024 117 / 89.)
+template <typename T, int N, int E, int W, int PS, int CL, int GMAX, int WPE>
+hipError_t launch_cols_occ(const PassArgs<T>& a, int mode, hipStream_t s) {
+  constexpr int TR = tile_rows(N), TC = tile_cols(N);
+  constexpr bool TILE_OK = (N / E) % TR == 0 && (W % TC == 0 || TC % W == 0);
+  const bool ok = occ_eligible(a, mode);
+  if ((a.flags & F_TILED) && (!ok || !TILE_OK)) return hipErrorInvalidValue;
   if constexpr (sizeof(T) == 4) {
     if (ok) {
       constexpr int threads = (N / E) * W;
       constexpr int SPF = N / W;
-      // the hoisted factor needs one set of optics for the whole call
-      const bool hoist = HOISTH != HOIST_NONE && a.fopt == nullptr;
-      static std::atomic<int> slot[2];
-      int slots = 0;
-      if constexpr (HOISTH != HOIST_NONE) {
-        if (hoist)
-          slots = cached_slots(slot[1], (const void*)&k_cols_pipe<T, N, E, W, PS, HOISTH, CL>, threads);
-      }
-      if (!hoist)
-        slots = cached_slots(slot[0], (const void*)&k_cols_pipe<T, N, E, W, PS, HOIST_NONE, CL>, threads);
-      int groups = slots / SPF;
-      if (groups < 1) groups = 1;
-      if (groups > a.batch) groups = a.batch;
-      int per = (a.batch + groups - 1) / groups;
-      if (per > kPipeMaxPer) per = kPipeMaxPer;
-      // at 4096 a field's 1024 strips already take four rounds of the resident
-      // workgroups: groups of at most 4 fields measured 800-811 us per 8 fields against
-      // 833-841 us for one group of 8 (2 fields: 797-813 us, 1 field: 830-841 us).  At
-      // 1024, where the groups of 8 fill one round, caps of 4 and 2 took 125 and 131 us
-      // against 115 us.
-      if constexpr (N >= 4096) {
-        if (per > 4) per = 4;
-      }
-      groups = (a.batch + per - 1) / per;
-      if constexpr (HOISTH != HOIST_NONE) {
-        if (hoist) {
-          k_cols_pipe<T, N, E, W, PS, HOISTH, CL><<<(unsigned)(groups * SPF), threads, 0, s>>>(a, per);
-          return hipGetLastError();
+      int per = 1;
+      if constexpr (GMAX > 1) {
+        if (a.fopt == nullptr) {
+          static std::atomic<int> slot{0};
+          const int slots = cached_slots(
+              slot, (const void*)&k_cols_occ<T, N, E, W, PS, CL, false, WPE>, threads);
+          int groups = slots / SPF;
+          if (groups < 1) groups = 1;
+          if (groups > a.batch) groups = a.batch;
+          per = (a.batch + groups - 1) / groups;
+          if (per > GMAX) per = GMAX;
         }
       }
-      k_cols_pipe<T, N, E, W, PS, HOIST_NONE, CL><<<(unsigned)(groups * SPF), threads, 0, s>>>(a, per);
+      const unsigned grid = (unsigned)((long long)((a.batch + per - 1) / per) * SPF);
+      if (a.flags & F_SPEC_OUT)
+        k_cols_occ<T, N, E, W, PS, CL, true, WPE><<<grid, threads, 0, s>>>(a, per);
+      else
+        k_cols_occ<T, N, E, W, PS, CL, false, WPE><<<grid, threads, 0, s>>>(a, per);
       return hipGetLastError();
     }
   }
-  return launch_cols<T, N, E, W, PS, false>(a, mode, s);
+  return launch_cols<T, N, E, W, PS>(a, mode, s);
+}
+
+// 1024 points: strips of 8 columns with 32 elements per thread (two transforms in two
+// passes each) once they fill the chip (512 resident workgroups), narrower strips of 4
+// with 16 elements below that: in place, 1 field 11.6 against 9.2 us, 4 fields 17.4
+// against 18.1, 32 fields 89 against 99.
+template <typename T, int N, int E, int W, int PS, int CL, int GMAX, int WPE, int E2, int W2,
+          int CL2, int WPE2>
+hipError_t launch_cols_pick(const PassArgs<T>& a, int mode, hipStream_t s) {
+  if (occ_eligible(a, mode) && (long long)a.batch * (N / W) < 512)
+    return launch_cols_occ<T, N, E2, W2, cmax(1, ilog2c(E2)), CL2, GMAX, WPE2>(a, mode, s);
+  return launch_cols_occ<T, N, E, W, PS, CL, GMAX, WPE>(a, mode, s);
 }
 
 // The fused complex64 propagation (transfer function / pupil / scale / spectrum
@@ -604,54 +492,41 @@ void add_row(Registry<T>& r) {
                               S::LINES, S::THREADS, S::LDS, S::LINES, 0};
 }
 
-template <typename T, int N, int E>
-void add_row_pipe(Registry<T>& r) {
-  using S = RowShape<T, N, E>;
+// One tile per workgroup, rows within waves (kind bit 3): LINES rows of N points.
+template <typename T, int N, int E, int LINES, int CL, int WPE>
+void add_row_occ(Registry<T>& r) {
+  constexpr int PS = cmax(1, ilog2c(E));
   constexpr int lg = ilog2c(N);
   int& k = r.nrows[lg];
   if (k >= kMaxVariants) return;
-  constexpr int lds = S::LDS + TwlLen<N, E>::value * (int)sizeof(cx<T>);
-  if constexpr (lds <= kLdsBudget)
-    r.rows[lg][k++] = RowVar<T>{&launch_rows_pipe<T, N, E, S::LINES, S::PS>,
-                                &launch_rows_grad<T, N, E, S::LINES, S::PS, (E <= 8)>, E,
-                                S::LINES, S::THREADS, lds, S::LINES, 2};
+  constexpr int lds = (LINES * RowPitch<N, PS, LINES>::value + TwlLen<N, E, CL>::value) *
+                      (int)sizeof(cx<T>);
+  static_assert(lds <= kLdsBudget, "LDS");
+  r.rows[lg][k++] = RowVar<T>{&launch_rows_occ<T, N, E, LINES, PS, CL, WPE>, nullptr, E, LINES,
+                              (N / E) * LINES, lds, LINES, 8};
 }
 
-// The plain row pass with LDS twiddles (kind bit 2), compact mode CL.
-template <typename T, int N, int E, int CL>
-void add_row_l(Registry<T>& r) {
-  using S = RowShape<T, N, E>;
-  constexpr int lg = ilog2c(N);
-  int& k = r.nrows[lg];
-  if (k >= kMaxVariants) return;
-  constexpr int lds = S::LDS + TwlLen<N, E, CL>::value * (int)sizeof(cx<T>);
-  if constexpr (lds <= kLdsBudget)
-    r.rows[lg][k++] = RowVar<T>{&launch_rows_l<T, N, E, S::LINES, S::PS, CL>,
-                                &launch_rows_grad<T, N, E, S::LINES, S::PS, (E <= 8)>, E,
-                                S::LINES, S::THREADS, lds, S::LINES, 4};
-}
-
-template <typename T, int N, int E, int WT, bool HOIST = false>
+template <typename T, int N, int E, int WT>
 void add_col(Registry<T>& r) {
   using S = ColShape<T, N, E, WT>;
   constexpr int lg = ilog2c(N);
   int& k = r.ncols[lg];
   if (k >= kMaxVariants) return;
-  r.cols[lg][k++] = ColVar<T>{&launch_cols<T, N, E, S::W, S::PS, HOIST>, E, S::W, S::THREADS,
-                              S::LDS, HOIST ? 1 : 0};
+  r.cols[lg][k++] = ColVar<T>{&launch_cols<T, N, E, S::W, S::PS>, E, S::W, S::THREADS,
+                              S::LDS, 0};
 }
 
-template <typename T, int N, int E, int WT, int HOISTH = HOIST_NONE, int CL = 0>
-void add_col_pipe(Registry<T>& r) {
-  using S = ColShape<T, N, E, WT>;
+template <typename T, int N, int E, int W, int CL, int GMAX, int WPE>
+void add_col_occ(Registry<T>& r) {
+  constexpr int PS = cmax(1, ilog2c(E));
   constexpr int lg = ilog2c(N);
   int& k = r.ncols[lg];
   if (k >= kMaxVariants) return;
-  constexpr int lds = S::LDS + TwlLen<N, E, CL>::value * (int)sizeof(cx<T>) +
-                      kPipeMaxPer * (int)sizeof(PipeField);
-  if constexpr (lds <= kLdsBudget)
-    r.cols[lg][k++] = ColVar<T>{&launch_cols_pipe<T, N, E, S::W, S::PS, HOISTH, CL>, E, S::W,
-                                S::THREADS, lds, HOISTH != HOIST_NONE ? 3 : 2};
+  constexpr int lds = (W * PaddedLen<N, PS>::value + TwlLen<N, E, CL>::value) *
+                      (int)sizeof(cx<T>);
+  static_assert(lds <= kLdsBudget, "LDS");
+  r.cols[lg][k++] = ColVar<T>{&launch_cols_occ<T, N, E, W, PS, CL, GMAX, WPE>, E, W,
+                              (N / E) * W, lds, 9};
 }
 
 template <typename T, int N>
@@ -664,6 +539,30 @@ void register_n(Registry<T>& r) {
   constexpr int WT = F32 ? 16 : 8;  // 128-byte row segments
   r.nrows[lg] = 0;
   r.ncols[lg] = 0;
+  // the schedules of complex64 by default (measured: see the bodies), then the plain ones
+  if constexpr (F32 && N == 256) {
+    add_row_occ<T, N, 8, 8, 0, 4>(r);
+    add_col_occ<T, N, 8, 8, 0, 4, 6>(r);
+    add_col_occ<T, N, 16, 8, 0, 4, 4>(r);
+  } else if constexpr (F32 && N == 512) {
+    add_row_occ<T, N, 8, 4, 0, 4>(r);
+    add_row_occ<T, N, 16, 8, 0, 3>(r);
+    add_col_occ<T, N, 8, 8, 0, 4, 6>(r);
+  } else if constexpr (F32 && N == 1024) {
+    add_row_occ<T, N, 16, 4, 0, 3>(r);
+    add_row_occ<T, N, 32, 8, 0, 2>(r);
+    add_col_occ<T, N, 32, 8, 0, 8, 2>(r);
+    r.cols[lg][0].fn = &launch_cols_pick<T, N, 32, 8, 5, 0, 8, 2, 16, 4, 3, 3>;
+    add_col_occ<T, N, 16, 4, 3, 8, 3>(r);
+  } else if constexpr (F32 && N == 2048) {
+    add_row_occ<T, N, 16, 2, 3, 4>(r);
+    add_col_occ<T, N, 32, 4, 4, 4, 2>(r);
+  } else if constexpr (F32 && N == 4096) {
+    // (the columns with the split tables: 10 spilled registers, 205 us for 2 fields
+    // against 152)
+    add_row_occ<T, N, 32, 2, 2, 2>(r);
+    add_col_occ<T, N, 32, 4, 1, 4, 2>(r);
+  }
   add_row<T, N, E0>(r);
   add_col<T, N, E0, WT>(r);
   if constexpr (E1 != E0 && N >= 16) {
@@ -672,26 +571,7 @@ void register_n(Registry<T>& r) {
   }
   if constexpr (N >= 256) {
     add_col<T, N, E0, WT / 2>(r);
-    if constexpr (F32) {
-      add_row<T, N, 32>(r);
-      add_col<T, N, 32, 16>(r);
-      add_col<T, N, 32, 8>(r);
-      add_col<T, N, 32, 8, true>(r);
-      add_col<T, N, 16, 8, true>(r);
-      add_col_pipe<T, N, 32, 8>(r);
-      add_col_pipe<T, N, 16, 8>(r);
-      add_col_pipe<T, N, 32, 4>(r);
-      add_col_pipe<T, N, 32, 8, HOIST_FACTOR>(r);
-      add_col_pipe<T, N, 16, 8, HOIST_PHASE>(r);
-      // the compact twiddle table lets 4-column strips of 4096 points pipeline (the
-      // hoisted factor does not fit in the registers beside them); at 2048 the split
-      // compact table brings 4-column strips to 77 KiB of LDS, two workgroups per CU
-      // (163 against 223 us per 8 fields)
-      if constexpr (N >= 4096) add_col_pipe<T, N, 32, 4, HOIST_NONE, true>(r);
-      if constexpr (N == 2048) add_col_pipe<T, N, 32, 4, HOIST_NONE, 2>(r);
-      add_row_pipe<T, N, 32>(r);
-      if constexpr (N == 4096) add_row_l<T, N, 32, 2>(r);
-    } else {
+    if constexpr (!F32) {
       add_row<T, N, 16>(r);
       add_col<T, N, 16, 8>(r);
     }

@@ -2,11 +2,13 @@
 //
 // Three tile shapes cover every operation:
 //   rows_body   LINES rows of one field: [spatial prologue] -> row FFT -> [epilogue]
+//               (rows_occ_body: the same with LDS twiddles and rows within waves)
 //   cols_body   W columns of one field:  [col FFT] -> [spectral middle] -> [col IFFT]
+//               (cols_occ_body: the fused complex64 pass, shared by groups of fields)
 //   small_body  a whole n x n field resident in LDS (n <= 128 for c64, <= 64 for c128):
 //               rows -> columns (+middle) -> rows, one HBM read and one HBM write.
-// The *_pipe_body variants run the same work over a sequence of fields or row tiles,
-// loading the next one while the current one is transformed.
+// The *_pipe_body variants run the same work over a sequence of fields, loading the next
+// one while the current one is transformed.
 // A field-to-field propagation of a large field is rows(fwd) -> cols(fwd,H,inv) ->
 // rows(inv): three sweeps over the field; the intermediate planes live in the output
 // buffer, so no workspace is needed (the adjoint can take one for its column pass).
@@ -43,16 +45,17 @@ enum : int {
 // of an n x n plane at
 //   (y/R)*R*n + (x/C)*R*C + (y%R)*C + x%C.
 // A block of R rows occupies the same addresses as in row-major order, so a row pass
-// over whole blocks converts in place; a column strip of width C then reads R*C
-// contiguous elements per block instead of C-element pieces of R different rows.  The
-// geometry follows each length's schedules (row tiles of R rows, strips of C columns):
-//   8 x 8 up to 2048 points: 512-byte chunks, every 128-byte line written whole by one
-//         store instruction (at 2048 the 4-column strips leave the plane row-major);
-//   2 x 4 at 4096: each 2-row block stays contiguous, so the 2-row passes keep their
-//         access pattern, and the 4-column strips read 64-byte chunks instead of 32.
-// (4 x 4 tiles at 2048 sped the column pass up by 25 us of 240, slowed each row pass
-// by about 10 us and doubled the adjoint's one-row gradient pass: not used.)
-constexpr int tile_rows(int n) { return n >= 4096 ? 2 : 8; }
+// over whole blocks converts in place; a column strip then reads R*C contiguous
+// elements per block instead of C-element pieces of R different rows.  One tile is one
+// 128-byte line: with the lines read whole, taller tiles gain the column pass nothing
+// (1024 points, 8 columns, traffic alone, 32 fields in place: 1 row 78 us, 2 rows 69,
+// 4 rows 68, 8 rows 67), and a block of two rows is what one wave of the row passes
+// holds, so that it converts without a workgroup barrier.
+//   2 x 8 up to 2048 points;
+//   2 x 4 at 4096, where the strips are 4 wide and read 64-byte pieces (4 x 4 tiles: the
+//   column pass 698 -> 630 us for 8 fields, the forward rows 390 -> 530, since a 2-row
+//   pass then writes half lines).
+constexpr int tile_rows(int) { return 2; }
 constexpr int tile_cols(int n) { return n >= 4096 ? 4 : 8; }
 
 // Offset of (y, x) in the block-tiled layout of an N-point plane.
@@ -78,24 +81,20 @@ struct TiledWaveMap {
   }
 };
 // Thread -> (row l, lane t) for a row tile of LINES rows that reads (or writes) the
-// block-tiled plane and writes (or reads) the natural one.  With 8 x 8 tiles and TL a
-// multiple of 16, each wave takes 4 rows x 16 lanes of an 8-row block: every access
-// of the tiled plane covers two 256-byte runs and every access of the natural plane
-// whole 128-byte lines (with 8 x 8 lanes per wave the two halves of a natural line
-// would come from two instructions, and the line would be written back twice).
-// Otherwise TiledWaveMap (whole tiles per instruction).
+// block-tiled plane and writes (or reads) the natural one.  NAT: a wave holds whole row
+// blocks with each row's TL threads consecutive (TL <= 64/TR), so the natural map
+// already covers whole tiles, and a block's data never leaves its wave.  Otherwise
+// TiledWaveMap (whole tiles per instruction, a row's threads over several waves).
 template <int N, int TL, int LINES>
 struct TiledRowMap {
   static constexpr int TR = tile_rows(N), TC = tile_cols(N);
   using WM = TiledWaveMap<TL, TR, TC>;
-  static constexpr bool LINE16 = TR == 8 && TC == 8 && TL % 16 == 0;
-  static constexpr bool ok = LINES % TR == 0 && TL % TC == 0 && (LINE16 || WM::ok);
+  static constexpr bool NAT = TL <= 64 && 64 % TL == 0 && (64 / TL) % TR == 0;
+  static constexpr bool ok = LINES % TR == 0 && TL % TC == 0 && (NAT || WM::ok);
   static __device__ __forceinline__ void map(int tid, int& l, int& t) {
-    if constexpr (LINE16) {
-      const int g = tid / (TR * TL), r = tid - g * (TR * TL);
-      const int wv = r >> 6, ln = r & 63;
-      l = g * TR + (ln >> 4) + 4 * (wv & 1);
-      t = (ln & 15) + 16 * (wv >> 1);
+    if constexpr (NAT) {
+      l = tid / TL;
+      t = tid - (tid / TL) * TL;
     } else {
       WM::map(tid, l, t);
     }
@@ -182,30 +181,28 @@ __device__ __forceinline__ T* uniform_ptr(T* p) {
   return (T*)(((uint64_t)hi << 32) | lo);
 }
 
-// Streaming accesses to field planes.  Every element of a plane is read once and
-// written once per sweep, and a sweep's planes are far larger than the caches, so the
-// loads and stores may carry the nontemporal hint (global_load/store ... nt).  A plain
-// 256 MiB copy runs at 6.0 TB/s without the hint and 6.4 TB/s with it on MI355X, but
-// the hint changes how the next sweep finds the plane, so it is chosen per access
-// site by measurement.  LP2D_NT is a mask of the sites that carry it.  Measured at
-// 32 x 1024^2 complex64: the row-pass loads gain 5-7 us per row pass and 8 us in the
-// following column pass, the gradient pass 28 us; the inverse row pass's stores (the
-// final field) leave the forward step unchanged and speed up the adjoint's column
-// pass (130 -> 124 us), the speckle chain (5 %) and the uneven batch (1.5 %).  Hinted
-// forward-row and column stores, and hinted column loads, were slower; the
-// whole-field kernels are indifferent.
+// Streaming accesses to field planes.  The nontemporal hint keeps what passes through
+// once (a call's input, its final field) from displacing the intermediate plane in the
+// Infinity Cache, where the next sweep finds it; an access that hits there is slower with
+// the hint (in place, 256 MB: 8.4 TB/s without, 6.2-6.9 with).  So it is chosen per access
+// site by measurement; LP2D_NT is a mask of the sites that carry it.  128 x 1024^2
+// complex64 in 256 MB chunks: as here 1049 us, forward-row loads without it 1151,
+// forward-row stores with it 1192, column stores with it 1195, inverse-row loads with it
+// 1092, inverse-row stores without it 1050 (the adjoint's column pass after them 130
+// against 124).
 enum : int {
-  NT_ROW_LD = 1,                   // row passes: loads
+  NT_ROW_LD = 1,                   // row passes: loads of the forward pass
   NT_ROW_ST = 2,                   //             stores of the forward pass
   NT_COL_LD = 4, NT_COL_ST = 8,    // column passes
   NT_GRAD = 16,                    // adjoint gradient row pass
   NT_SMALL = 32,                   // whole-field kernels
   NT_ROWI_ST = 64,                 // row passes: stores of the inverse pass
-  NT_TILE_ST = 128,                // whole-tile stores into the block-tiled plane
-                                   // (4096 points: LDS-twiddle rows, chained passes)
+  NT_TILE_ST = 128,                // chained passes: whole-tile stores at 4096 points
+  NT_ROWI_LD = 256,                // chained passes: loads
+  NT_OCCI_LD = 512,                // row passes: loads of the inverse pass
 };
 #ifndef LP2D_NT
-#define LP2D_NT (NT_ROW_LD | NT_GRAD | NT_ROWI_ST | NT_TILE_ST)
+#define LP2D_NT (NT_ROW_LD | NT_ROWI_LD | NT_GRAD | NT_ROWI_ST | NT_TILE_ST)
 #endif
 template <int SITE, typename T>
 __device__ __forceinline__ cx<T> gld(const LP2D_GLB cx<T>* p) {
@@ -234,11 +231,11 @@ __device__ __forceinline__ void gst(LP2D_GLB cx<T>* p, cx<T> x) {
 // whole 128-byte lines: the hint keeps a line out of the caches, so a line read in two
 // halves by two instructions is fetched twice (measured 1.23 x at 256 points, 8 lanes).
 template <typename T, int TL>
-constexpr int nt_row_site() { return TL * (int)sizeof(cx<T>) >= 128 ? NT_ROW_LD : 0; }
+constexpr int nt_row_site(int site = NT_ROW_LD) { return TL * (int)sizeof(cx<T>) >= 128 ? site : 0; }
 
 // The same rule for natural-order stores of a row pass: `run` lanes of one wave store
-// consecutive elements of a row (TL with the plain thread map; 16 or 64/tile_rows with
-// the tiled-plane maps).  A line written in two halves with the hint is written back
+// consecutive elements of a row (TL with the plain thread map, 64/tile_rows with the
+// tiled-plane map).  A line written in two halves with the hint is written back
 // twice (measured 1.088x at 256 points, 8 lanes), without it the halves merge in L2.
 template <typename T>
 constexpr int nt_store_site(int site, int run) {
@@ -246,7 +243,7 @@ constexpr int nt_store_site(int site, int run) {
 }
 template <int N, int TL, int LINES>
 constexpr int tiled_map_run() {
-  return TiledRowMap<N, TL, LINES>::LINE16 ? 16 : 64 / tile_rows(N);
+  return TiledRowMap<N, TL, LINES>::NAT ? TL : 64 / tile_rows(N);
 }
 
 // Base of field b's source / destination plane (b uniform across the workgroup).
@@ -563,48 +560,32 @@ struct RowPitch {
   static constexpr int value = PaddedLen<N, PS>::value + (LINES >= 8 ? 4 : 0);
 };
 
-// TW < 0: twiddles from the global tables; otherwise from the LDS tables twl of
-// twl_fill with compact mode TW, and a forward pass into the block-tiled plane takes
-// the whole-tile thread map with nontemporal stores (every store instruction writes
-// whole lines; the column pass then reads the plane faster: 786 -> 739 us at 8 x
-// 4096^2 for 22 us more here).  PHO (with FEAT off): the phase screen alone, applied
-// before the transform as the featured prologue applies it.
-template <typename T, int N, int E, int LINES, bool INV, int PS, bool FEAT = true, int TW = -1,
-          bool PHO = false>
+// Twiddles from the global tables; the exchanges synchronise the workgroup.
+template <typename T, int N, int E, int LINES, bool INV, int PS, bool FEAT = true>
 __device__ __forceinline__ void rows_body(const PassArgs<T>& a, int b, int y0, int nrows,
-                                          cx<T>* lds, int tid, const cx<T>* twl = nullptr) {
+                                          cx<T>* lds, int tid) {
   constexpr int TL = N / E;
   constexpr int L = RowPitch<N, PS, LINES>::value;
-  constexpr int TR = tile_rows(N), TC = tile_cols(N);
-  using WM = TiledWaveMap<TL, TR, TC>;
-  // Thread -> (row l, lane t).  Row-major planes: each row's TL threads consecutive.
-  // An inverse pass reading a block-tiled plane: each wave takes TR rows x 64/TR lanes,
-  // so every load instruction of the wave reads whole tiles (8 x 8: one 512-byte tile).
-  // (The same map for the forward pass of 2 x 4 tiles measured no different.)
-  int l = tid / TL, t = tid - (tid / TL) * TL;
-  if constexpr ((INV || TW >= 0) && TiledRowMap<N, TL, LINES>::ok) {
-    if (a.flags & F_TILED) TiledRowMap<N, TL, LINES>::map(tid, l, t);
-  }
+  constexpr unsigned TR = tile_rows(N);
+  // Thread -> (row l, lane t): each row's TL threads consecutive.
+  const int l = tid / TL, t = tid - (tid / TL) * TL;
   const int y = valid_row(y0 + l, y0 + nrows - 1);
   const bool valid = l < nrows;
   const long long frow = (long long)b * a.fstride + (long long)y * N;
-  // uniform base (SGPRs) + one 32-bit per-lane offset
+  // uniform base (SGPRs, the element stride in it) + one 32-bit per-lane offset; (y, x =
+  // t + TL*m) is at lo_n + TL*m in row-major order and at lo_t + TR*TL*m block-tiled (y0 a
+  // multiple of TR, TL of tile_cols)
+  const bool tiled = sizeof(T) == 4 && (a.flags & F_TILED) != 0;
   const long long ubase = (long long)y0 * N;
-  const unsigned lo = (unsigned)((y - y0) * N + t);
-  // block-tiled offset of (y, x = t + TL*m): lo_t + TR*TL*m (y0 a multiple of TR, TL of
-  // TC)
-  const bool tiled = (a.flags & F_TILED) != 0;
-  const unsigned lo_t = tiled_off<N>(l, t);
+  const unsigned lo_n = (unsigned)((y - y0) * N + t), lo_t = tiled_off<N>(y - y0, t);
+  const unsigned ld_o = (INV && tiled) ? lo_t : lo_n, st_o = (!INV && tiled) ? lo_t : lo_n;
+  const unsigned ld_s = (INV && tiled) ? TR * TL : TL, st_s = (!INV && tiled) ? TR * TL : TL;
   cx<T> v[E];
   const LP2D_GLB cx<T>* __restrict__ src = field_src(a, b) + ubase;
-  if (INV && tiled) {
 #pragma unroll
-    for (int m = 0; m < E; ++m) v[m] = gld<NT_ROW_LD>(src + (lo_t + (unsigned)(tile_rows(N) * TL * m)));
-  } else {
-#pragma unroll
-    for (int m = 0; m < E; ++m) v[m] = gld<nt_row_site<T, TL>()>(src + (lo + (unsigned)(TL * m)));
-  }
-  if constexpr (!FEAT && PHO) phase_mul_all<T, E, false>(a, v, b, y, t, TL, N);
+  for (int m = 0; m < E; ++m)
+    v[m] = gld<nt_row_site<T, TL>()>(
+        src + (size_t)(ld_s * (unsigned)m) + ld_o);
   if constexpr (FEAT) {
     if (a.flags & F_SPATIAL) {
       spatial_pro_all<T, E>(a, v, b, y, t, TL, N);
@@ -616,48 +597,87 @@ __device__ __forceinline__ void rows_body(const PassArgs<T>& a, int b, int y0, i
     }
   }
   LineAcc<T, PS> acc{lds + l * L};
-  if constexpr (TW >= 0)
-    line_fft_l<T, N, E, INV, TW>(v, t, acc, twl);
-  else
-    line_fft<T, N, E, INV>(v, t, acc, (INV ? a.tw_inv : a.tw) + (N - 2));
+  line_fft<T, N, E, INV>(v, t, acc, (INV ? a.tw_inv : a.tw) + (N - 2));
   LP2D_GLB cx<T>* __restrict__ dst = field_dst(a, b) + ubase;
-  // whole lines per store instruction: natural map / tiled-plane map
-  constexpr bool WN = nt_store_site<T>(1, TL) != 0;
-  constexpr bool WT =
-      nt_store_site<T>(1, (INV && TiledRowMap<N, TL, LINES>::ok) ? tiled_map_run<N, TL, LINES>()
-                                                                  : TL) != 0;
   if constexpr (FEAT) {
     spatial_epi_all<T, E>(a, v, b, y, t, TL, N, frow + t, valid);
-    if ((a.flags & F_NO_STORE) == 0) {
-      if (!INV && tiled) {
-#pragma unroll
-        for (int m = 0; m < E; ++m) gst<INV ? NT_ROWI_ST : NT_ROW_ST>(dst + (lo_t + (unsigned)(tile_rows(N) * TL * m)), v[m]);
-      } else if (tiled ? WT : WN) {
-#pragma unroll
-        for (int m = 0; m < E; ++m)
-          if (valid) gst<INV ? NT_ROWI_ST : NT_ROW_ST>(dst + (lo + (unsigned)(TL * m)), v[m]);
-      } else {
-#pragma unroll
-        for (int m = 0; m < E; ++m)
-          if (valid) gst<0>(dst + (lo + (unsigned)(TL * m)), v[m]);
-      }
-    }
+    if (a.flags & F_NO_STORE) return;
   } else {
     const T sc = (a.flags & F_SCALE) ? a.scale : (T)1;
-    if (!INV && tiled) {
 #pragma unroll
-      for (int m = 0; m < E; ++m)
-        gst<TW >= 0 ? NT_TILE_ST : NT_ROW_ST>(dst + (lo_t + (unsigned)(tile_rows(N) * TL * m)), mk(v[m].re * sc, v[m].im * sc));
-    } else if (tiled ? WT : WN) {
+    for (int m = 0; m < E; ++m) v[m] = cscale(v[m], sc);
+  }
 #pragma unroll
-      for (int m = 0; m < E; ++m)
-        if (valid) gst<INV ? NT_ROWI_ST : NT_ROW_ST>(dst + (lo + (unsigned)(TL * m)), mk(v[m].re * sc, v[m].im * sc));
-    } else {
+  for (int m = 0; m < E; ++m)
+    if (valid)
+      gst<INV ? nt_store_site<T>(NT_ROWI_ST, TL) : NT_ROW_ST>(
+          dst + (size_t)(st_s * (unsigned)m) + st_o, v[m]);
+}
+
+// The row pass of one whole tile of LINES rows per workgroup.  A row's TL threads are
+// consecutive; with TL <= 64 they lie in one wave, the exchanges of the transform
+// synchronise that wave only and no wave waits for another's loads.  Few elements per
+// thread: many waves are resident, and they overlap their loads, arithmetic and stores
+// without a prefetch.  Bound by memory traffic: 512 fields of 256 points in 64 us each
+// way, the time of a copy of the same bytes (the persistent pass with a prefetch:
+// 71-104 us).  The layouts are told apart by a uniform element stride and not by a
+// branch around the loads (two copies of them: 84 us), and the strides go into the
+// uniform base, so that one lane offset serves all E elements.  PHO: a forward pass
+// whose only feature is the phase screen; FEAT: every feature.
+template <typename T, int N, int E, int LINES, bool INV, int PS, bool FEAT, int CL, bool PHO>
+__device__ __forceinline__ void rows_occ_body(const PassArgs<T>& a, int b, int y0, cx<T>* lds,
+                                              const cx<T>* twl, int tid) {
+  constexpr int TL = N / E;
+  static_assert(N % LINES == 0 && (TL > 64 || 64 % TL == 0), "whole tiles, whole waves");
+  constexpr bool WS = TL <= 64;
+  constexpr int L = RowPitch<N, PS, LINES>::value;
+  constexpr unsigned TR = tile_rows(N);
+  const int l = tid / TL, t = tid - (tid / TL) * TL;
+  const int y = y0 + l;
+  const bool tiled = (a.flags & F_TILED) != 0;
+  const long long ubase = (long long)y0 * N;
+  // (y, x = t + TL*m): natural lo_n + TL*m, block-tiled lo_t + TR*TL*m
+  const unsigned lo_n = (unsigned)(l * N + t), lo_t = tiled_off<N>(l, t);
+  const unsigned ld_o = (INV && tiled) ? lo_t : lo_n, st_o = (!INV && tiled) ? lo_t : lo_n;
+  const unsigned ld_s = (INV && tiled) ? TR * TL : TL, st_s = (!INV && tiled) ? TR * TL : TL;
+  cx<T> v[E];
+  const LP2D_GLB cx<T>* __restrict__ src = field_src(a, b) + ubase;
 #pragma unroll
-      for (int m = 0; m < E; ++m)
-        if (valid) gst<0>(dst + (lo + (unsigned)(TL * m)), mk(v[m].re * sc, v[m].im * sc));
+  for (int m = 0; m < E; ++m)
+    v[m] = gld<INV ? NT_OCCI_LD : nt_row_site<T, TL>()>(src + (size_t)(ld_s * (unsigned)m) + ld_o);
+  if constexpr (PHO) phase_mul_all<T, E, false>(a, v, b, y, t, TL, N);
+  if constexpr (FEAT) {
+    if (a.flags & F_SPATIAL) {
+      spatial_pro_all<T, E>(a, v, b, y, t, TL, N);
+      if (a.flags & F_FIELD_OUT) {
+        LP2D_GLB cx<T>* fo =
+            glb(uniform_ptr(a.field_out + (long long)b * a.fstride)) + ubase;
+#pragma unroll
+        for (int m = 0; m < E; ++m) fo[lo_n + (unsigned)(TL * m)] = v[m];
+      }
     }
   }
+  LineAcc<T, PS> acc{lds + l * L};
+  line_fft_l<T, N, E, INV, CL, WS>(v, t, acc, twl);
+  if constexpr (WS && (64 / TL) % (int)TR != 0) {
+    // a row block over several waves, converted in place: its other waves may still have
+    // to load (a wave's own loads are complete once it has transformed them; with
+    // TL > 64 the barriers of the transform have seen to it)
+    if (tiled) __syncthreads();
+  }
+  LP2D_GLB cx<T>* __restrict__ dst = field_dst(a, b) + ubase;
+  if constexpr (FEAT) {
+    spatial_epi_all<T, E>(a, v, b, y, t, TL, N, (long long)b * a.fstride + (long long)y * N + t,
+                          true);
+    if (a.flags & F_NO_STORE) return;
+  } else {
+    const T sc = (a.flags & F_SCALE) ? a.scale : (T)1;
+#pragma unroll
+    for (int m = 0; m < E; ++m) v[m] = cscale(v[m], sc);
+  }
+#pragma unroll
+  for (int m = 0; m < E; ++m)
+    gst<INV ? nt_store_site<T>(NT_ROWI_ST, TL) : NT_ROW_ST>(dst + (size_t)(st_s * (unsigned)m) + st_o, v[m]);
 }
 
 // Chained planes (a multi-plane stack u_{k+1} = P(dz)[u_k exp(i phi_k)]): the inverse
@@ -687,7 +707,7 @@ __device__ __forceinline__ void rows_chain_body(const PassArgs<T>& a, int b, int
   cx<T> v[E];
   const LP2D_GLB cx<T>* __restrict__ src = field_src(a, b) + ubase;
 #pragma unroll
-  for (int m = 0; m < E; ++m) v[m] = gld<NT_ROW_LD>(src + (lo_t + TS * (unsigned)m));
+  for (int m = 0; m < E; ++m) v[m] = gld<NT_ROWI_LD>(src + (lo_t + TS * (unsigned)m));
   LineAcc<T, PS> acc{lds + l * L};
   if (twl)
     line_fft_l<T, N, E, true, CL>(v, t, acc, twl);
@@ -752,7 +772,7 @@ __device__ __forceinline__ void rows_adj_chain_body(const PassArgs<T>& a, int b0
     cx<T> v[E];
     const LP2D_GLB cx<T>* __restrict__ src = field_src(a, b) + ubase;
 #pragma unroll
-    for (int m = 0; m < E; ++m) v[m] = gld<NT_ROW_LD>(src + (lo_t + TS * (unsigned)m));
+    for (int m = 0; m < E; ++m) v[m] = gld<NT_ROWI_LD>(src + (lo_t + TS * (unsigned)m));
     if (twl)
       line_fft_l<T, N, E, true, CL>(v, tt, acc, twl);
     else
@@ -794,119 +814,6 @@ __device__ __forceinline__ void rows_adj_chain_body(const PassArgs<T>& a, int b0
 #pragma unroll
     for (int m = 0; m < E; ++m) partial[(long long)y * N + t + TL * m] = gsum[m];
   }
-}
-
-// Row tiles of LINES rows with software pipelining: the tile of step k+1 is loaded
-// into registers while tile k is transformed, as in the pipelined column pass.  A
-// workgroup takes tiles u0, u0 + ustep, u0 + 2*ustep, ... of the whole batch, so the
-// resident workgroups sweep the planes together.  Twiddles come from LDS (twl), so
-// nothing in the loop waits for the prefetch before it is needed.  Strided batches
-// of complex64 without spatial features, except (PH, forward pass) a phase screen:
-// its values are prefetched with the tile and applied before the next prefetch is
-// issued.  TILED: the forward pass stores, the inverse pass loads the block-tiled
-// layout.
-template <typename T, int N, int E, int LINES, bool INV, int PS, bool TILED, bool PH = false,
-          bool WSK = true>
-__device__ __forceinline__ void rows_pipe_body(const PassArgs<T>& a, int u0, int ustep,
-                                               int nunits, cx<T>* lds, const cx<T>* twl,
-                                               int tid) {
-  static_assert(sizeof(T) == 4, "complex64 path");
-  constexpr int TL = N / E;
-  constexpr int L = RowPitch<N, PS, LINES>::value;
-  constexpr int TPF = N / LINES;  // row tiles per field
-  static_assert(N % LINES == 0, "whole tiles");
-  constexpr int TR = tile_rows(N), TC = tile_cols(N);
-  using WM = TiledWaveMap<TL, TR, TC>;
-  static_assert(!TILED || (LINES % TR == 0 && TL % TC == 0), "tiled shape");
-  int l = tid / TL, t = tid - (tid / TL) * TL;
-  if constexpr (INV && TILED) {
-    if constexpr (TR == 8 && TC == 8 && TL % 16 == 0) {
-      // each wave takes 4 rows x 16 lanes of an 8-row block: every load instruction
-      // reads two 256-byte runs of the tiled plane, every store writes whole 128-byte
-      // lines of the natural one (with 8 x 8 lanes per wave the two halves of a line
-      // come from two waves, and the line is written back twice)
-      const int g = tid / (TR * TL), r = tid - g * (TR * TL);
-      const int wv = r >> 6, ln = r & 63;
-      l = g * TR + (ln >> 4) + 4 * (wv & 1);
-      t = (ln & 15) + 16 * (wv >> 1);
-    } else if constexpr (WM::ok) {
-      // TR rows x 64/TR lanes: every load instruction reads whole tiles
-      WM::map(tid, l, t);
-    }
-  }
-  // lane offsets inside a tile of LINES rows: natural (y, x) at y*N + x, tiled see
-  // F_TILED; element m of the thread is x = t + TL*m
-  const unsigned lo_n = (unsigned)(l * N + t);
-  const unsigned lo_t = tiled_off<N>(l, t);
-  constexpr bool LD_T = INV && TILED, ST_T = !INV && TILED;
-  const unsigned ld_o = LD_T ? lo_t : lo_n, st_o = ST_T ? lo_t : lo_n;
-  constexpr unsigned LD_S = LD_T ? TR * TL : TL, ST_S = ST_T ? TR * TL : TL;
-  // lanes of one wave storing consecutive elements of a natural-order row
-  constexpr int ST_RUN = (INV && TILED) ? ((TR == 8 && TC == 8 && TL % 16 == 0) ? 16
-                                           : WM::ok ? 64 / TR : TL)
-                                        : TL;
-  // each row's TL lanes in one wave (then the transform's exchanges synchronise one
-  // wave): the natural map up to 64 lanes, the tiled-plane maps when a wave holds
-  // whole rows.  Not for a layout conversion in place (WSK false): there the
-  // workgroup barriers inside the transform are what keep one wave's stores off
-  // data another wave of the workgroup has yet to load.
-  constexpr bool WS = WSK && TL <= 64 && 64 % TL == 0 &&
-                      (!(INV && TILED) ||
-                       ((TR == 8 && TC == 8 && TL % 16 == 0) ? TL == 16
-                        : WM::ok ? TL == 64 / TR : true));
-  LineAcc<T, PS> acc{lds + l * L};
-  const bool scale = (a.flags & F_SCALE) != 0;
-  auto tile_off = [&](int u) {
-    const int b = u / TPF;
-    return (long long)b * a.fstride + (long long)(u - b * TPF) * LINES * N;
-  };
-  // Step u moves tile u (prefetched by the previous step) from nxt into cur, requests
-  // tile u + ustep into nxt, then transforms cur and stores it; the first step is
-  // peeled so that the loop head's wait only ever covers the prefetch.
-  static_assert(!PH || !INV, "the screen is a forward-pass prologue");
-  cx<T> cur[E], nxt[E];
-  float phn[PH ? E : 1];
-  auto fetch = [&](int u) {
-    const LP2D_GLB cx<T>* __restrict__ src = glb(uniform_ptr(a.src + tile_off(u)));
-#pragma unroll
-    for (int m = 0; m < E; ++m)
-      nxt[m] = gld<LD_T ? NT_ROW_LD : nt_row_site<T, TL>()>(src + (ld_o + LD_S * (unsigned)m));
-    if constexpr (PH) {
-      const int b = u / TPF;
-      const LP2D_GLB float* __restrict__ ph =
-          glb(uniform_ptr(a.phase + (long long)b * a.phase_sb +
-                          (long long)(u - b * TPF) * LINES * N)) + lo_n;
-#pragma unroll
-      for (int m = 0; m < E; ++m) phn[m] = ph[TL * m];
-    }
-  };
-  auto step = [&](int u) {
-#pragma unroll
-    for (int m = 0; m < E; ++m) cur[m] = nxt[m];
-    if constexpr (PH) {  // x exp(i*phase): FP64 reduction to a fraction of a turn
-#pragma unroll
-      for (int m = 0; m < E; ++m) {
-        double r = (double)phn[m] * kInv2Pi;
-        r -= rint(r);
-        cur[m] = cmul(cur[m], exp_i_revolutions<T>(r));
-      }
-    }
-    if (u + ustep < nunits) fetch(u + ustep);  // uniform branch
-    line_fft_l<T, N, E, INV, 0, WS>(cur, t, acc, twl);
-    if (scale) {
-#pragma unroll
-      for (int m = 0; m < E; ++m) cur[m] = cscale(cur[m], a.scale);
-    }
-    LP2D_GLB cx<T>* __restrict__ dst = glb(uniform_ptr(a.dst + tile_off(u)));
-#pragma unroll
-    for (int m = 0; m < E; ++m)
-      gst<ST_T ? NT_ROW_ST : nt_store_site<T>(INV ? NT_ROWI_ST : NT_ROW_ST, ST_RUN)>(
-          dst + (st_o + ST_S * (unsigned)m), cur[m]);
-  };
-  if (u0 >= nunits) return;
-  fetch(u0);
-  step(u0);
-  for (int u = u0 + ustep; u < nunits; u += ustep) step(u);
 }
 
 // Thread -> (row l, lane t) of a gradient row tile of LINES rows.  Reading a
@@ -995,15 +902,10 @@ __device__ __forceinline__ void rows_grad_body(const PassArgs<T>& a, int b0, int
 // fastest, so every load/store instruction reads W*sizeof(cx) contiguous bytes from
 // each of 64/W rows.  lds: W * PaddedLen<N,PS> elements, interleaved by column.
 // MIDK selects the spectral stage compiled in: 0 none, 1 transfer function +
-// aperture + spectrum store, 2 everything (adds the mask multipliers), 3 as 1 with the
-// factor shared by a group of fields.
-// The workgroup runs fields [b0, b1) of the same strip in turn.  With MIDK == 3 the
-// spectral factor H(kx, ky) * aperture is the same for every field of the call, so it
-// is computed once per element before the field loop and kept in registers (2E more
-// live registers: a separate schedule for the autotuner to weigh).
+// aperture + spectrum store, 2 everything (adds the mask multipliers).
 template <typename T, int N, int E, int W, int MODE, int PS, int MIDK = 2>
-__device__ __forceinline__ void cols_body(const PassArgs<T>& a, int b0, int b1, int x0,
-                                          cx<T>* lds, int tid) {
+__device__ __forceinline__ void cols_body(const PassArgs<T>& a, int b, int x0, cx<T>* lds,
+                                          int tid) {
   constexpr int TL = N / E;
   const int c = tid % W, t = tid / W;
   const int x = x0 + c;
@@ -1011,61 +913,42 @@ __device__ __forceinline__ void cols_body(const PassArgs<T>& a, int b0, int b1, 
   InterAcc<T, PS, W> acc{lds + c};
   const bool mid = (a.flags & F_MID) != 0;
   const bool spec_out = (a.flags & F_SPEC_OUT) != 0;
-  cx<T> h[MIDK == 3 ? E : 1];
-  if constexpr (MIDK == 3) {  // (never used with per-field optics)
+  // uniform base (SGPRs, the element stride in it) + one 32-bit per-lane offset
+  cx<T> v[E];
+  const LP2D_GLB cx<T>* __restrict__ src = field_src(a, b) + x0;
 #pragma unroll
-    for (int m = 0; m < E; ++m)
-      h[m] = mid ? spectral_mid<T, false>(a, mk((T)1, (T)0), 0, t + TL * m, x, N)
-                 : mk((T)1, (T)0);
-  }
-  // Only the shared-factor class loops over fields: in the others a loop would let
-  // the compiler hoist the per-element factor out of it (all E values live at once).
-  const int bend = (MIDK == 3) ? b1 : b0 + 1;
-  for (int b = b0; b < bend; ++b) {
-    // uniform base (SGPRs) + one 32-bit per-lane offset: every load/store of the
-    // strip addresses as base + lane offset + compile-time constant
-    const long long ubase = (long long)b * a.fstride + x0;
-    cx<T> v[E];
-    // the shared-factor class never runs on per-field tables (their optics differ)
-    const LP2D_GLB cx<T>* __restrict__ src =
-        (MIDK == 3 ? glb(a.src + (long long)b * a.fstride) : field_src(a, b)) + x0;
+  for (int m = 0; m < E; ++m) v[m] = gld<NT_COL_LD>(src + (size_t)(TL * N) * m + lo);
+  if constexpr ((MODE & MODE_FWD) != 0) line_fft<T, N, E, false>(v, t, acc, a.tw + (N - 2));
+  if constexpr (MIDK == 1) {
+    if (mid) {
+      const PassArgs<T> ab = field_optics(a, b);
 #pragma unroll
-    for (int m = 0; m < E; ++m) v[m] = gld<NT_COL_LD>(src + (lo + (unsigned)(TL * N * m)));
-    if constexpr ((MODE & MODE_FWD) != 0) line_fft<T, N, E, false>(v, t, acc, a.tw + (N - 2));
-    if constexpr (MIDK == 3) {
-      if (mid) {
-#pragma unroll
-        for (int m = 0; m < E; ++m) v[m] = cmul(v[m], h[m]);
-      }
-    } else if constexpr (MIDK == 1) {
-      if (mid) {
-        const PassArgs<T> ab = field_optics(a, b);
-#pragma unroll
-        for (int m = 0; m < E; ++m) v[m] = spectral_mid<T, false>(ab, v[m], b, t + TL * m, x, N);
-      }
-    } else if constexpr (MIDK == 2) {
-      if (mid) {
-#pragma unroll
-        for (int m = 0; m < E; ++m) v[m] = spectral_mid<T, true>(a, v[m], b, t + TL * m, x, N);
-      }
+      for (int m = 0; m < E; ++m) v[m] = spectral_mid<T, false>(ab, v[m], b, t + TL * m, x, N);
     }
-    if constexpr (MIDK > 0) {
-      if (spec_out) {
+  } else if constexpr (MIDK == 2) {
+    if (mid) {
 #pragma unroll
-        for (int m = 0; m < E; ++m) a.spec_out[ubase + (lo + (unsigned)(TL * N * m))] = v[m];
-      }
+      for (int m = 0; m < E; ++m) v[m] = spectral_mid<T, true>(a, v[m], b, t + TL * m, x, N);
     }
-    // Keep the inverse transform's twiddle loads below the spectral stage: hoisted
-    // above it they stay live across it and cost registers.
-    asm volatile("" ::: "memory");
-    if constexpr ((MODE & MODE_INV) != 0)
-      line_fft<T, N, E, true>(v, t, acc, a.tw_inv + (N - 2));
-    LP2D_GLB cx<T>* __restrict__ dst =
-        (MIDK == 3 ? glb(a.dst + (long long)b * a.fstride) : field_dst(a, b)) + x0;
-    const T sc = (a.flags & F_SCALE) ? a.scale : (T)1;
-#pragma unroll
-    for (int m = 0; m < E; ++m) gst<NT_COL_ST>(dst + (lo + (unsigned)(TL * N * m)), mk(v[m].re * sc, v[m].im * sc));
   }
+  if constexpr (MIDK > 0) {
+    if (spec_out) {
+      LP2D_GLB cx<T>* __restrict__ so =
+          glb(uniform_ptr(a.spec_out + (long long)b * a.fstride + x0));
+#pragma unroll
+      for (int m = 0; m < E; ++m) gst<0>(so + (size_t)(TL * N) * m + lo, v[m]);
+    }
+  }
+  // Keep the inverse transform's twiddle loads below the spectral stage: hoisted
+  // above it they stay live across it and cost registers.
+  asm volatile("" ::: "memory");
+  if constexpr ((MODE & MODE_INV) != 0)
+    line_fft<T, N, E, true>(v, t, acc, a.tw_inv + (N - 2));
+  LP2D_GLB cx<T>* __restrict__ dst = field_dst(a, b) + x0;
+  const T sc = (a.flags & F_SCALE) ? a.scale : (T)1;
+#pragma unroll
+  for (int m = 0; m < E; ++m)
+    gst<NT_COL_ST>(dst + (size_t)(TL * N) * m + lo, mk(v[m].re * sc, v[m].im * sc));
 }
 
 // The gradient pass above, software-pipelined over the group's fields: the rows of
@@ -1224,131 +1107,79 @@ __device__ __forceinline__ void pipe_stage_fields(const PassArgs<T>& a, int b0, 
   }
 }
 
-// Column strips of a group of fields [b0, b1) with software pipelining: the strip of
-// field b+1 is loaded into registers while field b is transformed, so the memory
-// traffic of one field overlaps the arithmetic of the previous one instead of every
-// workgroup alternating between the two in step.  Twiddles come from LDS (twl) and
-// the fields' pointers and optics from pf, so that nothing in the loop waits for the
-// prefetch before it is needed.  Column FFT -> H, pupil -> column IFFT; complex64
-// only, evanescent modes pass through (EV_PASS), no mask multipliers.
-// Calls the pipelined class takes (host side): the fused forward+inverse pass of the
+// Calls the strips by occupancy take (host side): the fused forward+inverse pass of the
 // complex64 path without mask multipliers, evanescent modes passed through.
 template <typename T>
-inline bool pipe_eligible(const PassArgs<T>& a, int mode) {
+inline bool occ_eligible(const PassArgs<T>& a, int mode) {
   return sizeof(T) == 4 && mode == (MODE_FWD | MODE_INV) && a.evan == EV_PASS &&
          !(a.flags & (F_SMASK0 | F_SMASK1));
 }
 
-// HOISTH: the strip's transfer function is computed once, before the field loop, for
-// every field of the group (all fields of the call share one set of optics: a strided
-// batch without per-field tables).
-//   HOIST_FACTOR: exp(-2*pi*i*fr) x pupil held in registers (2E floats); the product
-//                 equals mid_fast's up to the sign of a zero.
-//   HOIST_PHASE:  only the FP64 part, the fractional phase fr and the pupil test, held
-//                 in registers (E floats and one bit mask); each field evaluates sin/cos
-//                 and the product is mid_fast's.
-// Measured per call (pipelined 8-column strips): 1024^2 x32 with 32 elements per thread
-// 118.9 us, factor 113.9, phase 121.8; 256^2 x64 with 16 elements 22.6 us, phase 20.2,
-// factor 22.2; 512^2 x64 with 16: 66.3, phase 62.0, factor 62.7.
-enum : int { HOIST_NONE = 0, HOIST_FACTOR = 1, HOIST_PHASE = 2 };
-template <typename T, int N, int E, int W, int PS, int HOISTH = HOIST_NONE, int CL = 0>
-__device__ __forceinline__ void cols_pipe_body(const PassArgs<T>& a, int b0, int b1, int x0,
-                                               cx<T>* lds, const cx<T>* twl,
-                                               const PipeField* pf, int tid) {
+// ----------------------------------------------------------------- column strips by occupancy
+// Column FFT -> H, pupil -> column IFFT of W-column strips of fields [b0, b1), without a
+// prefetch: few elements per thread and short tables keep several workgroups per CU,
+// which cover one another's loads and stores.  Complex64 calls of occ_eligible.
+// The strip's factor exp(-2*pi*i*fr) x pupil is computed before the loads and held in
+// registers (2E floats): for one field with its own optics (per-field tables), or for
+// all fields of the group (one set of optics).  A call without transfer function and
+// pupil multiplies by exactly one (col_mid).  The row stride goes into the uniform base,
+// so one lane offset serves all E elements: with an address per element the same
+// schedules spilled 10-100 registers and took 1.3-2 times as long.
+// In place, traffic alone / this pass / the pipelined strips it replaced (256 MB of
+// fields): 256 points 62 / 70 / 76 us, 512 61 / 78 / 86, 1024 67 / 89 / 113, 4096 (2
+// fields) - / 144 / 171; 2048 points, 3 fields in the flow 53 against 66.  (2048 points
+// with 16 elements per thread: 49 us with the last pass's twiddles as products of one
+// w^k, which costs precision, 64 with the tables that do not.)
+template <typename T, int N, int E, int W, int PS, int CL, bool SPEC>
+__device__ __forceinline__ void cols_occ_body(const PassArgs<T>& a, int b0, int b1, int x0,
+                                              cx<T>* lds, const cx<T>* twl, int tid) {
   static_assert(sizeof(T) == 4, "complex64 path");
   constexpr int TL = N / E;
   const int c = tid % W, t = tid / W;
   const int x = x0 + c;
   const int sx = x < N / 2 ? x : x - N;
-  // natural: (y, x) at y*N + x; block-tiled (W == tile_cols(N)): see F_TILED.  Row
-  // y = t + TL*m is at lo + TL*N*m in both (TL a multiple of tile_rows(N) when tiled).
-  const bool tiled = (a.flags & F_TILED) != 0;
-  const unsigned lo_n = (unsigned)(t * N + c);
-  const unsigned lo = tiled ? tiled_off<N>(t, c) : lo_n;
-  const int xoff = tiled ? (x0 / tile_cols(N)) * (tile_rows(N) * tile_cols(N)) : x0;
+  const unsigned lo_n = (unsigned)(t * N + x);
+  // row y = t + TL*m is TL*N*m further on in both layouts (TL a multiple of tile_rows(N)
+  // when tiled)
+  const unsigned lo = (a.flags & F_TILED) ? tiled_off<N>(t, x) : lo_n;
   InterAcc<T, PS, W> acc{lds + c};
-  const int flags = a.flags;
-  const bool mid = (flags & (F_H | F_APERTURE)) != 0;
-  const bool spec_out = (flags & F_SPEC_OUT) != 0;
-  const bool scale = (flags & F_SCALE) != 0;
-  // Step b moves field b's strip (prefetched by step b-1) from nxt into cur, requests
-  // field b+1 into nxt, then transforms cur and stores it.  The copy at the head of
-  // step b+1 therefore has exactly b's stores behind the loads it waits for, and the
-  // compiler's wait count lets those stores stay in flight.  The first step is peeled
-  // off the loop so that the loop head is only ever reached in that state (merged
-  // with the loop entry the wait would cover the stores as well).
-  cx<T> cur[E], nxt[E];
-  constexpr bool HF = HOISTH == HOIST_FACTOR, HP = HOISTH == HOIST_PHASE;
-  static_assert(!HP || E <= 32, "one mask bit per element");
-  cx<T> hm[HF ? E : 1];
-  float hfr[HP ? E : 1];
-  uint32_t hout = 0;
-  if constexpr (HF || HP) {
-    if (mid) {
-      const ColMid cm = col_mid(pf[0].o, flags, sx);
-#pragma unroll
-      for (int m = 0; m < E; ++m) {
-        bool out;
-        const float fr = mid_phase(cm, t + TL * m - (m >= E / 2 ? N : 0), out);
-        if constexpr (HF) {
-          hm[m] = mk(out ? 0.0f : __builtin_amdgcn_cosf(fr), out ? 0.0f : __builtin_amdgcn_sinf(fr));
-        } else {
-          hfr[m] = fr;
-          hout |= (uint32_t)out << m;
-        }
-      }
-    }
+  FieldOpt o;
+  if (a.fopt) {
+    o = a.fopt[b0];
+  } else {
+    o.k0sq = a.k0sq;
+    o.inv_ndL = a.inv_ndL;
+    o.z = a.z;
+    o.ap_r2 = a.ap_r2;
   }
-  auto fetch = [&](int bf) {
-    const LP2D_GLB cx<T>* __restrict__ src = glb(uniform_ptr((const cx<T>*)pf[bf - b0].src)) + xoff;
+  const ColMid cm = col_mid(o, a.flags, sx);
+  cx<T> hm[E];
 #pragma unroll
-    for (int m = 0; m < E; ++m) nxt[m] = gld<NT_COL_LD>(src + (lo + (unsigned)(TL * N * m)));
-  };
-  auto step = [&](int b) {
+  for (int m = 0; m < E; ++m) {
+    bool out;
+    const float fr = mid_phase(cm, t + TL * m - (m >= E / 2 ? N : 0), out);
+    hm[m] = mk(out ? 0.0f : __builtin_amdgcn_cosf(fr), out ? 0.0f : __builtin_amdgcn_sinf(fr));
+  }
+  const T sc = (a.flags & F_SCALE) ? a.scale : (T)1;
+  for (int b = b0; b < b1; ++b) {
+    cx<T> v[E];
+    const LP2D_GLB cx<T>* __restrict__ src = field_src(a, b);
 #pragma unroll
-    for (int m = 0; m < E; ++m) cur[m] = nxt[m];
-    if (b + 1 < b1) fetch(b + 1);  // uniform branch
-    line_fft_l<T, N, E, false, CL>(cur, t, acc, twl);
-    if (HF && mid) {
+    for (int m = 0; m < E; ++m) v[m] = gld<NT_COL_LD>(src + (size_t)(TL * N) * m + lo);
+    line_fft_l<T, N, E, false, CL>(v, t, acc, twl);
 #pragma unroll
-      for (int m = 0; m < E; ++m) cur[m] = cmulc(cur[m], hm[HF ? m : 0]);
-    } else if (HP && mid) {
+    for (int m = 0; m < E; ++m) v[m] = cmulc(v[m], hm[m]);
+    if constexpr (SPEC) {
+      LP2D_GLB cx<T>* __restrict__ so = glb(uniform_ptr(a.spec_out + (long long)b * a.fstride));
 #pragma unroll
-      for (int m = 0; m < E; ++m) {
-        const float fr = hfr[HP ? m : 0];
-        const cx<float> r = cmulc(cur[m], mk(__builtin_amdgcn_cosf(fr), __builtin_amdgcn_sinf(fr)));
-        const bool out = (hout >> m) & 1u;
-        cur[m] = mk(out ? 0.0f : r.re, out ? 0.0f : r.im);
-      }
-    } else if (mid) {
-      ColMid cm = col_mid(pf[b - b0].o, flags, sx);
-      // opaque per field: otherwise the per-element frequencies (the same for every
-      // field of a strip) are hoisted out of the field loop and held for all E
-      // elements at once
-      int tt = t;
-      asm volatile("" : "+v"(cm.c0), "+v"(cm.fx2), "+v"(cm.inv_ndL), "+v"(tt));
-      // fftfreq order: index t + TL*m is a negative frequency for m >= E/2
-#pragma unroll
-      for (int m = 0; m < E; ++m) cur[m] = mid_fast(cm, cur[m], tt + TL * m - (m >= E / 2 ? N : 0));
+      for (int m = 0; m < E; ++m) gst<NT_COL_ST>(so + (size_t)(TL * N) * m + lo_n, v[m]);
     }
-    if (spec_out) {
-      LP2D_GLB cx<T>* __restrict__ so = glb(a.spec_out + (long long)b * a.fstride + x0);
+    line_fft_l<T, N, E, true, CL>(v, t, acc, twl);
+    LP2D_GLB cx<T>* __restrict__ dst = field_dst(a, b);
 #pragma unroll
-      for (int m = 0; m < E; ++m) gst<NT_COL_ST>(so + (lo_n + (unsigned)(TL * N * m)), cur[m]);
-    }
-    line_fft_l<T, N, E, true, CL>(cur, t, acc, twl);
-    if (scale) {
-#pragma unroll
-      for (int m = 0; m < E; ++m) cur[m] = cscale(cur[m], a.scale);
-    }
-    LP2D_GLB cx<T>* __restrict__ dst = glb(uniform_ptr((cx<T>*)pf[b - b0].dst)) + xoff;
-#pragma unroll
-    for (int m = 0; m < E; ++m) gst<NT_COL_ST>(dst + (lo + (unsigned)(TL * N * m)), cur[m]);
-  };
-  if (b0 >= b1) return;  // (the launchers size the groups so that none is empty)
-  fetch(b0);
-  step(b0);
-  for (int b = b0 + 1; b < b1; ++b) step(b);
+    for (int m = 0; m < E; ++m)
+      gst<NT_COL_ST>(dst + (size_t)(TL * N) * m + lo, cscale(v[m], sc));
+  }
 }
 
 // ----------------------------------------------------------------- whole field in LDS

@@ -30,15 +30,14 @@ struct RowVar {
   RowGradLaunch<T> grad_fn;  // adjoint last pass with the batch-summed phase gradient
   int E, lines, threads, lds;
   int grad_lines;  // row tile of grad_fn: whole 8-row blocks where the threads allow
-  int kind;        // bit 1: software-pipelined over the row tiles of the batch
-                   // bit 2: twiddles staged in LDS, one resident round of workgroups
+  int kind;        // bit 3: one tile per workgroup, LDS twiddles, no global tables
 };
 template <typename T>
 struct ColVar {
   ColLaunch<T> fn;
   int E, W, threads, lds;
   int kind;  // bit 0: transfer function computed once per group of fields (shared-H)
-             // bit 1: software-pipelined over the fields of a group
+             // bit 3: the fused complex64 pass by occupancy, reads block-tiled planes
 };
 template <typename T>
 struct SmallVar {
