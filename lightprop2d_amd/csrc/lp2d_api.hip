@@ -368,11 +368,10 @@ const RowVar<T>& grad_variant(int lg) {
 // it (whole blocks again, unless it stores nothing).
 template <typename T>
 int tiled_flag(const PassArgs<T>& cols_a, int lg, bool grad = false, bool grad_store = true) {
-  if (sizeof(T) != 4) return 0;
   const int n = 1 << lg;
   const ColVar<T>& cv = reg<T>()->cols[lg][sel_of(dt<T>(), 1, lg)];
   const RowVar<T>& rv = reg<T>()->rows[lg][sel_of(dt<T>(), 0, lg)];
-  const int tr = tile_rows(n), tc = tile_cols(n);
+  const int tr = tile_rows(n), tc = tile_cols<T>(n);
   if (!(cv.kind & 8) || (n / cv.E) % tr != 0) return 0;
   if (cv.W % tc != 0 && tc % cv.W != 0) return 0;
   if (!occ_eligible(cols_a, MODE_FWD | MODE_INV)) return 0;

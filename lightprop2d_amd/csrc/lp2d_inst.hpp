@@ -204,7 +204,7 @@ inline int cached_slots(std::atomic<int>& slot, const void* kernel, int threads)
 
 template <typename T, int N, int E, int LINES, int PS>
 hipError_t launch_rows(const PassArgs<T>& a, bool inv, hipStream_t s) {
-  if ((a.flags & F_TILED) && (LINES % tile_rows(N) != 0 || (N / E) % tile_cols(N) != 0))
+  if ((a.flags & F_TILED) && (LINES % tile_rows(N) != 0 || (N / E) % tile_cols<T>(N) != 0))
     return hipErrorInvalidValue;
   constexpr int threads = (N / E) * LINES;
   constexpr int TPF = (N + LINES - 1) / LINES;
@@ -227,7 +227,7 @@ hipError_t launch_rows(const PassArgs<T>& a, bool inv, hipStream_t s) {
 // One tile per workgroup, rows within waves; every feature and the per-field tables.
 template <typename T, int N, int E, int LINES, int PS, int CL, int WPE>
 hipError_t launch_rows_occ(const PassArgs<T>& a, bool inv, hipStream_t s) {
-  if ((a.flags & F_TILED) && (LINES % tile_rows(N) != 0 || (N / E) % tile_cols(N) != 0))
+  if ((a.flags & F_TILED) && (LINES % tile_rows(N) != 0 || (N / E) % tile_cols<T>(N) != 0))
     return hipErrorInvalidValue;
   constexpr int threads = (N / E) * LINES;
   const unsigned grid = (unsigned)((long long)a.batch * (N / LINES));
@@ -253,7 +253,7 @@ hipError_t launch_rows_grad(const PassArgs<T>& a, int groups, float* partial, hi
   const bool in_place = (const void*)a.src == (const void*)a.dst;
   if ((a.flags & F_TILED) &&
       (((LINES % tile_rows(N)) != 0 && !(a.flags & F_NO_STORE) && in_place) ||
-       (N / E) % tile_cols(N) != 0))
+       (N / E) % tile_cols<T>(N) != 0))
     return hipErrorInvalidValue;
   constexpr int threads = (N / E) * LINES;
   constexpr int TPF = (N + LINES - 1) / LINES;
@@ -268,7 +268,7 @@ hipError_t launch_rows_grad(const PassArgs<T>& a, int groups, float* partial, hi
 // the plain sweeps.
 template <typename T, int N, int E, int LINES, int PS>
 constexpr bool chain_ok() {
-  return sizeof(T) == 4 && N % LINES == 0 && TiledRowMap<N, N / E, LINES>::ok;
+  return sizeof(T) == 4 && N % LINES == 0 && TiledRowMap<T, N, N / E, LINES>::ok;
 }
 template <typename T, int N, int E, int LINES, int PS, int WPE = 2>
 hipError_t launch_rows_chain(const PassArgs<T>& a, hipStream_t s) {
@@ -400,34 +400,32 @@ hipError_t launch_cols(const PassArgs<T>& a, int mode, hipStream_t s) {
 // 256 points 81 / 70 us, 512 84 / 78, 1024 117 / 89.)
 template <typename T, int N, int E, int W, int PS, int CL, int GMAX, int WPE>
 hipError_t launch_cols_occ(const PassArgs<T>& a, int mode, hipStream_t s) {
-  constexpr int TR = tile_rows(N), TC = tile_cols(N);
+  constexpr int TR = tile_rows(N), TC = tile_cols<T>(N);
   constexpr bool TILE_OK = (N / E) % TR == 0 && (W % TC == 0 || TC % W == 0);
   const bool ok = occ_eligible(a, mode);
   if ((a.flags & F_TILED) && (!ok || !TILE_OK)) return hipErrorInvalidValue;
-  if constexpr (sizeof(T) == 4) {
-    if (ok) {
-      constexpr int threads = (N / E) * W;
-      constexpr int SPF = N / W;
-      int per = 1;
-      if constexpr (GMAX > 1) {
-        if (a.fopt == nullptr) {
-          static std::atomic<int> slot{0};
-          const int slots = cached_slots(
-              slot, (const void*)&k_cols_occ<T, N, E, W, PS, CL, false, WPE>, threads);
-          int groups = slots / SPF;
-          if (groups < 1) groups = 1;
-          if (groups > a.batch) groups = a.batch;
-          per = (a.batch + groups - 1) / groups;
-          if (per > GMAX) per = GMAX;
-        }
+  if (ok) {
+    constexpr int threads = (N / E) * W;
+    constexpr int SPF = N / W;
+    int per = 1;
+    if constexpr (GMAX > 1) {
+      if (a.fopt == nullptr) {
+        static std::atomic<int> slot{0};
+        const int slots = cached_slots(
+            slot, (const void*)&k_cols_occ<T, N, E, W, PS, CL, false, WPE>, threads);
+        int groups = slots / SPF;
+        if (groups < 1) groups = 1;
+        if (groups > a.batch) groups = a.batch;
+        per = (a.batch + groups - 1) / groups;
+        if (per > GMAX) per = GMAX;
       }
-      const unsigned grid = (unsigned)((long long)((a.batch + per - 1) / per) * SPF);
-      if (a.flags & F_SPEC_OUT)
-        k_cols_occ<T, N, E, W, PS, CL, true, WPE><<<grid, threads, 0, s>>>(a, per);
-      else
-        k_cols_occ<T, N, E, W, PS, CL, false, WPE><<<grid, threads, 0, s>>>(a, per);
-      return hipGetLastError();
     }
+    const unsigned grid = (unsigned)((long long)((a.batch + per - 1) / per) * SPF);
+    if (a.flags & F_SPEC_OUT)
+      k_cols_occ<T, N, E, W, PS, CL, true, WPE><<<grid, threads, 0, s>>>(a, per);
+    else
+      k_cols_occ<T, N, E, W, PS, CL, false, WPE><<<grid, threads, 0, s>>>(a, per);
+    return hipGetLastError();
   }
   return launch_cols<T, N, E, W, PS>(a, mode, s);
 }
@@ -539,7 +537,7 @@ void register_n(Registry<T>& r) {
   constexpr int WT = F32 ? 16 : 8;  // 128-byte row segments
   r.nrows[lg] = 0;
   r.ncols[lg] = 0;
-  // the schedules of complex64 by default (measured: see the bodies), then the plain ones
+  // the default schedules (measured: see the bodies), then the plain ones
   if constexpr (F32 && N == 256) {
     add_row_occ<T, N, 8, 8, 0, 4>(r);
     add_col_occ<T, N, 8, 8, 0, 4, 6>(r);
@@ -563,6 +561,31 @@ void register_n(Registry<T>& r) {
     add_row_occ<T, N, 32, 2, 2, 2>(r);
     add_col_occ<T, N, 32, 4, 1, 4, 2>(r);
   }
+  // complex128, a propagation with the plain passes and these: 512 fields of 128 points
+  // 141 -> 128 us, 64 of 256 84 -> 74, 16 of 512 91 -> 78, 5 of 1024 119 -> 101, 2 of
+  // 2048 210 -> 161.  At 4096
+  // points a row of 2-row tiles takes a CU's whole LDS (133-158 us against 109 of the
+  // plain pass with 16 elements per thread), so the plane stays row-major and only the
+  // columns change: 479 -> 430.
+  if constexpr (!F32 && N == 256) {
+    add_row_occ<T, N, 8, 4, 0, 3>(r);
+    add_col_occ<T, N, 8, 4, 0, 4, 3>(r);
+  } else if constexpr (!F32 && N == 512) {
+    add_row_occ<T, N, 8, 2, 0, 3>(r);
+    add_col_occ<T, N, 8, 4, 0, 4, 3>(r);
+  } else if constexpr (!F32 && N == 1024) {
+    add_row_occ<T, N, 8, 2, 3, 4>(r);
+    add_col_occ<T, N, 16, 4, 3, 4, 2>(r);
+  } else if constexpr (!F32 && N == 2048) {
+    add_row_occ<T, N, 16, 2, 3, 2>(r);
+    add_col_occ<T, N, 16, 2, 3, 4, 2>(r);
+  } else if constexpr (!F32 && N == 4096) {
+    add_row<T, N, 16>(r);
+    add_col_occ<T, N, 32, 2, 3, 4, 1>(r);
+  } else if constexpr (!F32 && N == 128) {
+    add_row_occ<T, N, 8, 4, 0, 3>(r);
+    add_col_occ<T, N, 8, 4, 0, 4, 3>(r);
+  }
   add_row<T, N, E0>(r);
   add_col<T, N, E0, WT>(r);
   if constexpr (E1 != E0 && N >= 16) {
@@ -572,7 +595,7 @@ void register_n(Registry<T>& r) {
   if constexpr (N >= 256) {
     add_col<T, N, E0, WT / 2>(r);
     if constexpr (!F32) {
-      add_row<T, N, 16>(r);
+      if constexpr (N != 4096) add_row<T, N, 16>(r);
       add_col<T, N, 16, 8>(r);
     }
   }

@@ -54,14 +54,18 @@ enum : int {
 //   2 x 8 up to 2048 points;
 //   2 x 4 at 4096, where the strips are 4 wide and read 64-byte pieces (4 x 4 tiles: the
 //   column pass 698 -> 630 us for 8 fields, the forward rows 390 -> 530, since a 2-row
-//   pass then writes half lines).
+//   pass then writes half lines);
+//   2 x 4 in complex128 (4096 points keep the natural layout there, see register_n).
 constexpr int tile_rows(int) { return 2; }
-constexpr int tile_cols(int n) { return n >= 4096 ? 4 : 8; }
+template <typename T>
+constexpr int tile_cols(int n) {
+  return sizeof(T) == 8 || n >= 4096 ? 4 : 8;
+}
 
 // Offset of (y, x) in the block-tiled layout of an N-point plane.
-template <int N>
+template <typename T, int N>
 __device__ __forceinline__ unsigned tiled_off(int y, int x) {
-  constexpr unsigned R = tile_rows(N), C = tile_cols(N);
+  constexpr unsigned R = tile_rows(N), C = tile_cols<T>(N);
   const unsigned uy = (unsigned)y, ux = (unsigned)x;
   return (uy / R) * R * N + (ux / C) * (R * C) + (uy % R) * C + ux % C;
 }
@@ -85,9 +89,9 @@ struct TiledWaveMap {
 // blocks with each row's TL threads consecutive (TL <= 64/TR), so the natural map
 // already covers whole tiles, and a block's data never leaves its wave.  Otherwise
 // TiledWaveMap (whole tiles per instruction, a row's threads over several waves).
-template <int N, int TL, int LINES>
+template <typename T, int N, int TL, int LINES>
 struct TiledRowMap {
-  static constexpr int TR = tile_rows(N), TC = tile_cols(N);
+  static constexpr int TR = tile_rows(N), TC = tile_cols<T>(N);
   using WM = TiledWaveMap<TL, TR, TC>;
   static constexpr bool NAT = TL <= 64 && 64 % TL == 0 && (64 / TL) % TR == 0;
   static constexpr bool ok = LINES % TR == 0 && TL % TC == 0 && (NAT || WM::ok);
@@ -241,9 +245,9 @@ template <typename T>
 constexpr int nt_store_site(int site, int run) {
   return run * (int)sizeof(cx<T>) >= 128 ? site : 0;
 }
-template <int N, int TL, int LINES>
+template <typename T, int N, int TL, int LINES>
 constexpr int tiled_map_run() {
-  return TiledRowMap<N, TL, LINES>::NAT ? TL : 64 / tile_rows(N);
+  return TiledRowMap<T, N, TL, LINES>::NAT ? TL : 64 / tile_rows(N);
 }
 
 // Base of field b's source / destination plane (b uniform across the workgroup).
@@ -575,9 +579,9 @@ __device__ __forceinline__ void rows_body(const PassArgs<T>& a, int b, int y0, i
   // uniform base (SGPRs, the element stride in it) + one 32-bit per-lane offset; (y, x =
   // t + TL*m) is at lo_n + TL*m in row-major order and at lo_t + TR*TL*m block-tiled (y0 a
   // multiple of TR, TL of tile_cols)
-  const bool tiled = sizeof(T) == 4 && (a.flags & F_TILED) != 0;
+  const bool tiled = (a.flags & F_TILED) != 0;
   const long long ubase = (long long)y0 * N;
-  const unsigned lo_n = (unsigned)((y - y0) * N + t), lo_t = tiled_off<N>(y - y0, t);
+  const unsigned lo_n = (unsigned)((y - y0) * N + t), lo_t = tiled_off<T, N>(y - y0, t);
   const unsigned ld_o = (INV && tiled) ? lo_t : lo_n, st_o = (!INV && tiled) ? lo_t : lo_n;
   const unsigned ld_s = (INV && tiled) ? TR * TL : TL, st_s = (!INV && tiled) ? TR * TL : TL;
   cx<T> v[E];
@@ -637,7 +641,7 @@ __device__ __forceinline__ void rows_occ_body(const PassArgs<T>& a, int b, int y
   const bool tiled = (a.flags & F_TILED) != 0;
   const long long ubase = (long long)y0 * N;
   // (y, x = t + TL*m): natural lo_n + TL*m, block-tiled lo_t + TR*TL*m
-  const unsigned lo_n = (unsigned)(l * N + t), lo_t = tiled_off<N>(l, t);
+  const unsigned lo_n = (unsigned)(l * N + t), lo_t = tiled_off<T, N>(l, t);
   const unsigned ld_o = (INV && tiled) ? lo_t : lo_n, st_o = (!INV && tiled) ? lo_t : lo_n;
   const unsigned ld_s = (INV && tiled) ? TR * TL : TL, st_s = (!INV && tiled) ? TR * TL : TL;
   cx<T> v[E];
@@ -695,14 +699,14 @@ __device__ __forceinline__ void rows_chain_body(const PassArgs<T>& a, int b, int
                                                 cx<T>* lds, const cx<T>* twl, int tid) {
   constexpr int TL = N / E;
   constexpr int L = RowPitch<N, PS, LINES>::value;
-  constexpr int TR = tile_rows(N), TC = tile_cols(N);
-  using RM = TiledRowMap<N, TL, LINES>;
+  constexpr int TR = tile_rows(N), TC = tile_cols<T>(N);
+  using RM = TiledRowMap<T, N, TL, LINES>;
   static_assert(RM::ok && N % LINES == 0, "whole tiles of whole row blocks");
   int l, t;
   RM::map(tid, l, t);
   const int y = y0 + l;
   const long long ubase = (long long)y0 * N;
-  const unsigned lo_t = tiled_off<N>(l, t);
+  const unsigned lo_t = tiled_off<T, N>(l, t);
   constexpr unsigned TS = TR * TL;  // tiled offset step of element m
   cx<T> v[E];
   const LP2D_GLB cx<T>* __restrict__ src = field_src(a, b) + ubase;
@@ -720,7 +724,7 @@ __device__ __forceinline__ void rows_chain_body(const PassArgs<T>& a, int b, int
         glb(uniform_ptr(a.field_out + (long long)b * a.fstride)) + (long long)y * N;
 #pragma unroll
     for (int m = 0; m < E; ++m)
-      gst<nt_store_site<T>(NT_ROWI_ST, tiled_map_run<N, TL, LINES>())>(ck + (t + TL * m), v[m]);
+      gst<nt_store_site<T>(NT_ROWI_ST, tiled_map_run<T, N, TL, LINES>())>(ck + (t + TL * m), v[m]);
   }
   phase_mul_all<T, E, false>(a, v, b, y, t, TL, N);
   if (twl)
@@ -751,13 +755,13 @@ __device__ __forceinline__ void rows_adj_chain_body(const PassArgs<T>& a, int b0
   constexpr int TL = N / E;
   constexpr int L = RowPitch<N, PS, LINES>::value;
   constexpr int TR = tile_rows(N);
-  using RM = TiledRowMap<N, TL, LINES>;
+  using RM = TiledRowMap<T, N, TL, LINES>;
   static_assert(RM::ok && N % LINES == 0, "whole tiles of whole row blocks");
   int l, t;
   RM::map(tid, l, t);
   const int y = y0 + l;
   const long long ubase = (long long)y0 * N;
-  const unsigned lo_t = tiled_off<N>(l, t);
+  const unsigned lo_t = tiled_off<T, N>(l, t);
   constexpr unsigned TS = TR * TL;
   const bool store = (a.flags & F_NO_STORE) == 0;
   LineAcc<T, PS> acc{lds + l * L};
@@ -794,7 +798,7 @@ __device__ __forceinline__ void rows_adj_chain_body(const PassArgs<T>& a, int b0
         LP2D_GLB cx<T>* __restrict__ dst = field_dst(a, b) + (long long)y * N;
 #pragma unroll
         for (int m = 0; m < E; ++m)
-          gst<nt_store_site<T>(NT_ROWI_ST, tiled_map_run<N, TL, LINES>())>(dst + (t + TL * m),
+          gst<nt_store_site<T>(NT_ROWI_ST, tiled_map_run<T, N, TL, LINES>())>(dst + (t + TL * m),
                                                                           v[m]);
       }
     } else {
@@ -864,7 +868,7 @@ __device__ __forceinline__ void rows_grad_body(const PassArgs<T>& a, int b0, int
   }
   // block-tiled offset of (y, x = t + TL*m) in the field: lo_t + R*TL*m (TL a multiple
   // of C); any row tile height can read it, storing in place needs whole blocks
-  const unsigned lo_t = tiled_off<N>(y, t);
+  const unsigned lo_t = tiled_off<T, N>(y, t);
   for (int b = b0; b < b1; ++b) {
     const long long frow = (long long)b * a.fstride + (long long)y * N;
     cx<T> v[E];
@@ -977,7 +981,7 @@ __device__ __forceinline__ void rows_grad_pipe_body(const PassArgs<T>& a, int b0
     gsum[m] = 0.f;
   }
   const unsigned lo_n = (unsigned)(y * N + t);
-  const unsigned lo_t = tiled_off<N>(y, t);
+  const unsigned lo_t = tiled_off<T, N>(y, t);
   cx<T> cur[E], nxt[E], ucur[E], unxt[E];
   auto fetch = [&](int bf) {
     const LP2D_GLB cx<T>* __restrict__ src = glb(a.src + (long long)bf * a.fstride);
@@ -1077,6 +1081,26 @@ __device__ __forceinline__ float mid_phase(const ColMid& m, int sy, bool& out) {
   return kz_frac_fast(m.c0 - fy2, m.z);
 }
 
+// The conjugate of H(fy) * pupil(fy) at signed frequency index sy of the column: in
+// complex128 with the operations of spectral_mid.
+template <typename T>
+__device__ __forceinline__ cx<T> mid_factor(const ColMid& m, int sy) {
+#pragma clang fp contract(off)
+  if constexpr (sizeof(T) == 4) {
+    bool out;
+    const float fr = mid_phase(m, sy, out);
+    return mk(out ? 0.0f : __builtin_amdgcn_cosf(fr), out ? 0.0f : __builtin_amdgcn_sinf(fr));
+  } else {
+    const double fy = (double)sy * m.inv_ndL;
+    const double fy2 = fy * fy;
+    const double kz2 = m.c0 - fy2;
+    const double d = sqrt(kz2 > 0.0 ? kz2 : 0.0) * m.z;
+    const cx<double> h = expi_rev(d - trunc(d));
+    const bool out = m.fx2 + fy2 > m.ap;
+    return mk(out ? 0.0 : h.re, out ? 0.0 : h.im);
+  }
+}
+
 // One field of a pipelined column group, staged in LDS at kernel start so that the
 // field loop reads its pointers and optics without global loads (a global load there
 // would wait behind the prefetch and the previous field's stores).
@@ -1107,20 +1131,20 @@ __device__ __forceinline__ void pipe_stage_fields(const PassArgs<T>& a, int b0, 
   }
 }
 
-// Calls the strips by occupancy take (host side): the fused forward+inverse pass of the
-// complex64 path without mask multipliers, evanescent modes passed through.
+// Calls the strips by occupancy take (host side): the fused forward+inverse pass without
+// mask multipliers, evanescent modes passed through.
 template <typename T>
 inline bool occ_eligible(const PassArgs<T>& a, int mode) {
-  return sizeof(T) == 4 && mode == (MODE_FWD | MODE_INV) && a.evan == EV_PASS &&
+  return mode == (MODE_FWD | MODE_INV) && a.evan == EV_PASS &&
          !(a.flags & (F_SMASK0 | F_SMASK1));
 }
 
 // ----------------------------------------------------------------- column strips by occupancy
 // Column FFT -> H, pupil -> column IFFT of W-column strips of fields [b0, b1), without a
 // prefetch: few elements per thread and short tables keep several workgroups per CU,
-// which cover one another's loads and stores.  Complex64 calls of occ_eligible.
+// which cover one another's loads and stores.  Calls of occ_eligible.
 // The strip's factor exp(-2*pi*i*fr) x pupil is computed before the loads and held in
-// registers (2E floats): for one field with its own optics (per-field tables), or for
+// registers (E numbers): for one field with its own optics (per-field tables), or for
 // all fields of the group (one set of optics).  A call without transfer function and
 // pupil multiplies by exactly one (col_mid).  The row stride goes into the uniform base,
 // so one lane offset serves all E elements: with an address per element the same
@@ -1130,10 +1154,12 @@ inline bool occ_eligible(const PassArgs<T>& a, int mode) {
 // fields) - / 144 / 171; 2048 points, 3 fields in the flow 53 against 66.  (2048 points
 // with 16 elements per thread: 49 us with the last pass's twiddles as products of one
 // w^k, which costs precision, 64 with the tables that do not.)
+// Complex128, where computing the factor is the greater part of the arithmetic, this pass
+// / the plain one: 64 fields of 256 points 31 / 36 us, 16 of 512 34 / 42, 5 of 1024
+// 43 / 54, 2 of 2048 72 / 107, 1 of 4096 225 / 266.
 template <typename T, int N, int E, int W, int PS, int CL, bool SPEC>
 __device__ __forceinline__ void cols_occ_body(const PassArgs<T>& a, int b0, int b1, int x0,
                                               cx<T>* lds, const cx<T>* twl, int tid) {
-  static_assert(sizeof(T) == 4, "complex64 path");
   constexpr int TL = N / E;
   const int c = tid % W, t = tid / W;
   const int x = x0 + c;
@@ -1141,7 +1167,7 @@ __device__ __forceinline__ void cols_occ_body(const PassArgs<T>& a, int b0, int 
   const unsigned lo_n = (unsigned)(t * N + x);
   // row y = t + TL*m is TL*N*m further on in both layouts (TL a multiple of tile_rows(N)
   // when tiled)
-  const unsigned lo = (a.flags & F_TILED) ? tiled_off<N>(t, x) : lo_n;
+  const unsigned lo = (a.flags & F_TILED) ? tiled_off<T, N>(t, x) : lo_n;
   InterAcc<T, PS, W> acc{lds + c};
   FieldOpt o;
   if (a.fopt) {
@@ -1155,11 +1181,7 @@ __device__ __forceinline__ void cols_occ_body(const PassArgs<T>& a, int b0, int 
   const ColMid cm = col_mid(o, a.flags, sx);
   cx<T> hm[E];
 #pragma unroll
-  for (int m = 0; m < E; ++m) {
-    bool out;
-    const float fr = mid_phase(cm, t + TL * m - (m >= E / 2 ? N : 0), out);
-    hm[m] = mk(out ? 0.0f : __builtin_amdgcn_cosf(fr), out ? 0.0f : __builtin_amdgcn_sinf(fr));
-  }
+  for (int m = 0; m < E; ++m) hm[m] = mid_factor<T>(cm, t + TL * m - (m >= E / 2 ? N : 0));
   const T sc = (a.flags & F_SCALE) ? a.scale : (T)1;
   for (int b = b0; b < b1; ++b) {
     cx<T> v[E];
