@@ -293,8 +293,8 @@ __device__ __forceinline__ void line_fft(cx<T> (&v)[E], int t, const Acc& acc,
 // 2.5 KB for n = 2048 with 16 elements per thread).  Every twiddle is one product of two
 // table entries, where the product tree multiplies the error of w^k by r: n = 2048,
 // whole propagation against 64 bits 4.3e-7 with the tree, 3.0e-7 with the full table.
-// CL = 4 (half compact, a last pass of radix 2): w^k for k < NS/2, the other half being
-// w^k = -i * w^{k - NS/2} exactly.
+// CL = 4 (quarter table): w^j for j < N/4; w^{rk} is the entry at r*k mod N/4 turned by the
+// quarter turns of r*k, exactly.
 constexpr int twl_radix(int N, int E, int ns) { return N / ns >= E ? E : N / ns; }
 constexpr bool twl_compact(int N, int E, int ns, int CL) {
   return CL != 0 && ns > 1 && ns * twl_radix(N, E, ns) == N &&
@@ -306,7 +306,7 @@ constexpr int twl_split(int ns) {
   return 1 << (l / 2);
 }
 constexpr int twl_compact_len(int ns, int R, int CL) {
-  if (CL == 4) return ns / 2;
+  if (CL == 4) return ns * R / 4;
   return CL >= 2 ? (twl_split(ns) + ns / twl_split(ns)) * (CL == 3 ? R + 2 : 1) : ns;
 }
 constexpr int twl_off(int N, int E, int NS, int CL = 0) {
@@ -353,8 +353,7 @@ __device__ __forceinline__ void twl_fill(cx<T>* twl, const cx<T>* __restrict__ t
           twl, tw, tid, [](int i) { return (L - 2) + (i < S ? i : (i - S) * S); },
           [](int i) { return OFF + i; });
     } else if constexpr (twl_compact(N, E, NS, CL) && CL == 4) {
-      static_assert(R == 2, "half table");
-      twl_copy<T, NS / 2, THREADS>(
+      twl_copy<T, L / 4, THREADS>(
           twl, tw, tid, [](int i) { return (L - 2) + i; }, [](int i) { return OFF + i; });
     } else if constexpr (twl_compact(N, E, NS, CL) && CL == 3) {
       // rows w^{r*i}, i < S, then w^{r*S*h}, h < NS/S (r < R; an entry is in the table:
@@ -399,10 +398,18 @@ __device__ __forceinline__ void stockham_l(cx<T> (&v)[E], int t, const Acc& acc,
 #pragma unroll
     for (int r = 0; r < R; ++r) a[r] = v[q + r * B];
     if constexpr (twl_compact(N, E, NS, CL) && CL == 4) {
-      const cx<T> q = twl[twl_off(N, E, NS, CL) + (k & (NS / 2 - 1))];
-      const bool rot = k >= NS / 2;
-      const cx<T> w = mk(rot ? q.im : q.re, rot ? -q.re : q.im);
-      a[1] = INV ? cmulc(a[1], w) : cmul(a[1], w);
+      const cx<T>* tp = twl + twl_off(N, E, NS, CL);
+#pragma unroll
+      for (int r = 1; r < R; ++r) {
+        const int i = r * k;
+        cx<T> w = tp[i & (N / 4 - 1)];
+        if (4 * r > R) {  // otherwise r*k < N/4
+          const int q = i / (N / 4);
+          const T x = (q & 1) ? w.im : w.re, y = (q & 1) ? w.re : w.im;
+          w = mk(q >= 2 ? -x : x, (q == 1 || q == 2) ? -y : y);  // (-i)^q
+        }
+        a[r] = INV ? cmulc(a[r], w) : cmul(a[r], w);
+      }
     } else if constexpr (twl_compact(N, E, NS, CL) && CL == 3) {
       constexpr int S = twl_split(NS), OFF = twl_off(N, E, NS, CL), P = R + 2;
       const cx<T>* ta = twl + (OFF + (k & (S - 1)) * P);

@@ -547,11 +547,14 @@ void register_n(Registry<T>& r) {
     add_row_occ<T, N, 16, 8, 0, 3>(r);
     add_col_occ<T, N, 8, 8, 0, 4, 6>(r);
   } else if constexpr (F32 && N == 1024) {
-    add_row_occ<T, N, 16, 4, 0, 3>(r);
+    // (the quarter table leaves room for four workgroups per CU instead of three with the
+    // full one: 4 fields, one round of 1024 workgroups, 50.4 -> 44.6 us; 32 fields 262 ->
+    // 260)
+    add_row_occ<T, N, 16, 4, 4, 4>(r);
     add_row_occ<T, N, 32, 8, 0, 2>(r);
     add_col_occ<T, N, 32, 8, 0, 8, 2>(r);
-    r.cols[lg][0].fn = &launch_cols_pick<T, N, 32, 8, 5, 0, 8, 2, 16, 4, 3, 3>;
-    add_col_occ<T, N, 16, 4, 3, 8, 3>(r);
+    r.cols[lg][0].fn = &launch_cols_pick<T, N, 32, 8, 5, 0, 8, 2, 16, 4, 4, 3>;
+    add_col_occ<T, N, 16, 4, 4, 8, 3>(r);
   } else if constexpr (F32 && N == 2048) {
     add_row_occ<T, N, 16, 2, 3, 4>(r);
     add_col_occ<T, N, 32, 4, 4, 4, 2>(r);
@@ -562,7 +565,7 @@ void register_n(Registry<T>& r) {
     add_col_occ<T, N, 32, 4, 1, 4, 2>(r);
   }
   // complex128, a propagation with the plain passes and these: 512 fields of 128 points
-  // 141 -> 128 us, 64 of 256 84 -> 74, 16 of 512 91 -> 78, 5 of 1024 119 -> 101, 2 of
+  // 141 -> 128 us, 64 of 256 84 -> 74, 16 of 512 91 -> 76, 5 of 1024 119 -> 100, 2 of
   // 2048 210 -> 161.  At 4096
   // points a row of 2-row tiles takes a CU's whole LDS (133-158 us against 109 of the
   // plain pass with 16 elements per thread), so the plane stays row-major and only the
@@ -572,10 +575,10 @@ void register_n(Registry<T>& r) {
     add_col_occ<T, N, 8, 4, 0, 4, 3>(r);
   } else if constexpr (!F32 && N == 512) {
     add_row_occ<T, N, 8, 2, 0, 3>(r);
-    add_col_occ<T, N, 8, 4, 0, 4, 3>(r);
+    add_col_occ<T, N, 8, 4, 4, 4, 4>(r);
   } else if constexpr (!F32 && N == 1024) {
     add_row_occ<T, N, 8, 2, 3, 4>(r);
-    add_col_occ<T, N, 16, 4, 3, 4, 2>(r);
+    add_col_occ<T, N, 16, 4, 4, 4, 2>(r);
   } else if constexpr (!F32 && N == 2048) {
     add_row_occ<T, N, 16, 2, 3, 2>(r);
     add_col_occ<T, N, 16, 2, 3, 4, 2>(r);
