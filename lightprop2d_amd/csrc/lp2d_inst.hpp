@@ -81,31 +81,17 @@ __global__ __launch_bounds__((N / E) * LINES) LP2D_OCC void k_rows_grad(PassArgs
 
 // Chained-plane row pass: one workgroup per row tile of LINES rows of one field.
 // WPE: waves per SIMD the register budget is sized for.
-template <typename T, int N, int E, int LINES, int PS, int WPE>
+template <typename T, int N, int E, int LINES, int PS, int CL, int WPE>
 __global__ __launch_bounds__((N / E) * LINES) __attribute__((amdgpu_waves_per_eu(WPE)))
 void k_rows_chain(PassArgs<T> a) {
   __shared__ cx<T> lds[LINES * RowPitch<N, PS, LINES>::value];
-  constexpr int TPF = N / LINES;
-  const int tile = blockIdx.x;
-  const int b = tile / TPF;
-  rows_chain_body<T, N, E, LINES, PS>(a, b, (tile - b * TPF) * LINES, lds, nullptr,
-                                      threadIdx.x);
-}
-
-// The same with the twiddles staged once in LDS (compact last pass when CL), each
-// workgroup taking every gridDim.x-th row tile of the batch (one resident round).
-template <typename T, int N, int E, int LINES, int PS, int WPE, int CL>
-__global__ __launch_bounds__((N / E) * LINES) __attribute__((amdgpu_waves_per_eu(WPE)))
-void k_rows_chain_l(PassArgs<T> a, int nunits) {
-  __shared__ cx<T> lds[LINES * RowPitch<N, PS, LINES>::value];
   __shared__ cx<T> twl[TwlLen<N, E, CL>::value];
+  constexpr int TPF = N / LINES;
   twl_fill<T, N, E, (N / E) * LINES, 1, CL>(twl, a.tw, threadIdx.x);
   __syncthreads();
-  constexpr int TPF = N / LINES;
-  for (int u = blockIdx.x; u < nunits; u += gridDim.x) {
-    const int b = u / TPF;
-    rows_chain_body<T, N, E, LINES, PS, CL>(a, b, (u - b * TPF) * LINES, lds, twl, threadIdx.x);
-  }
+  const int tile = blockIdx.x;
+  const int b = tile / TPF;
+  rows_chain_body<T, N, E, LINES, PS, CL>(a, b, (tile - b * TPF) * LINES, lds, twl, threadIdx.x);
 }
 
 // Grid: (N/W strips) x fields.
@@ -262,99 +248,43 @@ hipError_t launch_rows_grad(const PassArgs<T>& a, int groups, float* partial, hi
   return hipGetLastError();
 }
 
-// The chained-plane pass runs on block-tiled planes of whole tiles only (complex64
-// schedules whose row tile is a whole number of row blocks and whose threads cover
-// whole tile widths); other shapes report hipErrorInvalidValue and the caller runs
-// the plain sweeps.
-template <typename T, int N, int E, int LINES, int PS>
-constexpr bool chain_ok() {
-  return sizeof(T) == 4 && N % LINES == 0 && TiledRowMap<T, N, N / E, LINES>::ok;
-}
-template <typename T, int N, int E, int LINES, int PS, int WPE = 2>
+// The chained-plane passes run on block-tiled planes only.
+template <typename T, int N, int E, int LINES, int PS, int CL, int WPE>
 hipError_t launch_rows_chain(const PassArgs<T>& a, hipStream_t s) {
-  if constexpr (chain_ok<T, N, E, LINES, PS>()) {
-    if (!(a.flags & F_TILED) || !a.phase || a.src_tab || a.dst_tab) return hipErrorInvalidValue;
-    constexpr int threads = (N / E) * LINES;
-    const unsigned grid = (unsigned)((long long)a.batch * (N / LINES));
-    k_rows_chain<T, N, E, LINES, PS, WPE><<<grid, threads, 0, s>>>(a);
-    return hipGetLastError();
-  } else {
-    (void)a;
-    (void)s;
-    return hipErrorInvalidValue;
-  }
+  if (!(a.flags & F_TILED) || !a.phase || a.src_tab || a.dst_tab) return hipErrorInvalidValue;
+  constexpr int threads = (N / E) * LINES;
+  const unsigned grid = (unsigned)((long long)a.batch * (N / LINES));
+  k_rows_chain<T, N, E, LINES, PS, CL, WPE><<<grid, threads, 0, s>>>(a);
+  return hipGetLastError();
 }
 
-// Adjoint chained pass: grid (N/LINES row tiles) x (field groups); twiddles in LDS
-// (TWL) or from the global tables.
-template <typename T, int N, int E, int LINES, int PS, int CL, bool TWL, bool LAST, int WPE = 2>
+// Adjoint chained pass: grid (N/LINES row tiles) x (field groups).
+template <typename T, int N, int E, int LINES, int PS, int CL, bool LAST, int WPE>
 __global__ __launch_bounds__((N / E) * LINES) __attribute__((amdgpu_waves_per_eu(WPE)))
 void k_rows_adj_chain(PassArgs<T> a, int groups, float* partial) {
   __shared__ cx<T> lds[LINES * RowPitch<N, PS, LINES>::value];
-  __shared__ cx<T> twl[TWL ? TwlLen<N, E, CL>::value : 1];
+  __shared__ cx<T> twl[TwlLen<N, E, CL>::value];
   constexpr int TPF = N / LINES;
   const int tile = blockIdx.x % TPF, g = blockIdx.x / TPF;
   const int per = (a.batch + groups - 1) / groups;
   const int b0 = g * per, b1 = cmin(a.batch, b0 + per);
-  if constexpr (TWL) {
-    twl_fill<T, N, E, (N / E) * LINES, 1, CL>(twl, a.tw, threadIdx.x);
-    __syncthreads();
-  }
+  twl_fill<T, N, E, (N / E) * LINES, 1, CL>(twl, a.tw, threadIdx.x);
+  __syncthreads();
   rows_adj_chain_body<T, N, E, LINES, PS, CL, LAST>(
-      a, b0, b1, tile * LINES, partial ? partial + (long long)g * N * N : nullptr, lds,
-      TWL ? twl : nullptr, threadIdx.x);
+      a, b0, b1, tile * LINES, partial ? partial + (long long)g * N * N : nullptr, lds, twl,
+      threadIdx.x);
 }
 
-template <typename T, int N, int E, int LINES, int CL>
-constexpr int chain_l_lds() {
-  return (LINES * RowPitch<N, cmax(1, ilog2c(E)), LINES>::value + TwlLen<N, E, CL>::value) *
-         (int)sizeof(cx<T>);
-}
-template <typename T, int N, int E, int LINES, int PS, int WPE, int CL>
-hipError_t launch_rows_chain_l(const PassArgs<T>& a, hipStream_t s) {
-  if constexpr (chain_ok<T, N, E, LINES, PS>() && chain_l_lds<T, N, E, LINES, CL>() <= kLdsBudget) {
-    if (!(a.flags & F_TILED) || !a.phase || a.src_tab || a.dst_tab) return hipErrorInvalidValue;
-    constexpr int threads = (N / E) * LINES;
-    const long long units = (long long)a.batch * (N / LINES);
-    if (units > 0x7fffffff) return hipErrorInvalidValue;
-    static std::atomic<int> slot{0};
-    const int slots = cached_slots(slot, (const void*)&k_rows_chain_l<T, N, E, LINES, PS, WPE, CL>,
-                                   threads);
-    const int grid = (int)(units < slots ? units : slots);
-    k_rows_chain_l<T, N, E, LINES, PS, WPE, CL><<<grid, threads, 0, s>>>(a, (int)units);
-    return hipGetLastError();
-  } else {
-    (void)a;
-    (void)s;
-    return hipErrorInvalidValue;
-  }
-}
-
-template <typename T, int N, int E, int LINES, int CL, bool TWL>
-constexpr int adj_chain_lds() {
-  return (LINES * RowPitch<N, cmax(1, ilog2c(E)), LINES>::value +
-          (TWL ? TwlLen<N, E, CL>::value : 0)) *
-         (int)sizeof(cx<T>);
-}
-template <typename T, int N, int E, int LINES, int PS, int CL, bool TWL, bool LAST, int WPE = 2>
+template <typename T, int N, int E, int LINES, int PS, int CL, bool LAST, int WPE>
 hipError_t launch_rows_adj_chain(const PassArgs<T>& a, int groups, float* partial, hipStream_t s) {
-  if constexpr (chain_ok<T, N, E, LINES, PS>() &&
-                adj_chain_lds<T, N, E, LINES, CL, TWL>() <= kLdsBudget) {
-    if (!(a.flags & F_TILED) || !a.phase || (partial && !a.u_saved) || a.src_tab || a.dst_tab ||
-        groups < 1)
-      return hipErrorInvalidValue;
-    constexpr int threads = (N / E) * LINES;
-    const long long grid = (long long)(N / LINES) * groups;
-    k_rows_adj_chain<T, N, E, LINES, PS, CL, TWL, LAST, WPE><<<(unsigned)grid, threads, 0, s>>>(
-        a, groups, partial);
-    return hipGetLastError();
-  } else {
-    (void)a;
-    (void)groups;
-    (void)partial;
-    (void)s;
+  if (!(a.flags & F_TILED) || !a.phase || (partial && !a.u_saved) || a.src_tab || a.dst_tab ||
+      groups < 1)
     return hipErrorInvalidValue;
-  }
+  constexpr int threads = (N / E) * LINES;
+  const long long grid = (long long)(N / LINES) * groups;
+  k_rows_adj_chain<T, N, E, LINES, PS, CL, LAST, WPE><<<(unsigned)grid, threads, 0, s>>>(
+      a, groups, partial);
+  return hipGetLastError();
 }
 
 template <typename T, int N, int E, int W, int PS>
@@ -527,6 +457,26 @@ void add_col_occ(Registry<T>& r) {
                               (N / E) * W, lds, 9};
 }
 
+template <typename T, int N, int E, int LINES, int CL, int WPE>
+void add_chain(Registry<T>& r) {
+  constexpr int PS = cmax(1, ilog2c(E));
+  constexpr int lg = ilog2c(N);
+  const int k = r.nchain[lg]++;
+  r.chain[lg][k] = &launch_rows_chain<T, N, E, LINES, PS, CL, WPE>;
+  r.chain_E[lg][k] = E;
+  r.chain_lines[lg][k] = LINES;
+}
+
+template <typename T, int N, int E, int LINES, int CL, int WPE>
+void set_adj_chain(Registry<T>& r) {
+  constexpr int PS = cmax(1, ilog2c(E));
+  constexpr int lg = ilog2c(N);
+  r.adj_chain[lg][0] = &launch_rows_adj_chain<T, N, E, LINES, PS, CL, false, WPE>;
+  r.adj_chain[lg][1] = &launch_rows_adj_chain<T, N, E, LINES, PS, CL, true, WPE>;
+  r.adj_threads[lg] = (N / E) * LINES;
+  r.adj_lines[lg] = LINES;
+}
+
 template <typename T, int N>
 void register_n(Registry<T>& r) {
   constexpr int lg = ilog2c(N);
@@ -602,100 +552,34 @@ void register_n(Registry<T>& r) {
       add_col<T, N, 16, 8>(r);
     }
   }
-  // chained-plane row pass: 32 elements per thread in the row pass's shape (2 waves
-  // per SIMD) with global or LDS-staged twiddles, and 16 elements per thread in row
-  // tiles of at least one tile height (4 waves per SIMD).  Variant 0 is the fastest
-  // measured per size (stack of 5 screens, per pass; 32 global / 32 LDS / 16):
-  // 4096 x8: 680 / 627 / 846 us; 1024 x32: 142 / 117 / 148; 512 x64: 67 / 63 / 81;
-  // 256 x128: 36 / 34 / 33.  At 4096 the 2-row tiles with the split compact table
-  // (75 KiB of LDS, two workgroups per CU) take 529 us and come first.
+  // chained-plane row passes of the stack (the first is the default; the other, forward
+  // with 5 screens: 128 x 256^2 310 / 309 us and 8 x 256^2 68 / 72, 64 x 512^2 545 / 565,
+  // 32 x 1024^2 1055 / 1116, 8 x 2048^2 1432 / 1530, 8 x 4096^2 6329 / 6339, 4096^2 862 /
+  // 890) and its adjoint, where 16 elements per thread leave room for the group's
+  // gradient sums
   r.nchain[lg] = 0;
-  for (int k = 0; k < 4; ++k) r.chain_twl[lg][k] = 0;
   r.adj_chain[lg][0] = r.adj_chain[lg][1] = nullptr;
   r.adj_threads[lg] = r.adj_lines[lg] = 0;
-  if constexpr (F32 && N >= 256) {
-    using S = RowShape<T, N, 32>;
-    constexpr int L16 = cmax(tile_rows(N), 256 / (N / 16));
-    constexpr int PS16 = cmax(1, ilog2c(16));
-    constexpr bool ok32 = chain_ok<T, N, 32, S::LINES, S::PS>();
-    constexpr bool ok16 = (N / 16) * L16 <= 1024 && chain_ok<T, N, 16, L16, PS16>();
-    auto add32 = [&] {
-      if constexpr (ok32) {
-        const int k = r.nchain[lg]++;
-        r.chain[lg][k] = &launch_rows_chain<T, N, 32, S::LINES, S::PS, 2>;
-        r.chain_E[lg][k] = 32;
-        r.chain_lines[lg][k] = S::LINES;
-      }
-    };
-    auto add16 = [&] {
-      if constexpr (ok16) {
-        const int k = r.nchain[lg]++;
-        r.chain[lg][k] = &launch_rows_chain<T, N, 16, L16, PS16, 4>;
-        r.chain_E[lg][k] = 16;
-        r.chain_lines[lg][k] = L16;
-      }
-    };
-    // twiddles in LDS: the 32-element shape (rows of the row pass, or 4 rows at 4096
-    // with the compact last-pass table: one 512-thread workgroup per CU)
-    constexpr int LL = N >= 4096 ? 4 : S::LINES;
-    constexpr int CLL = N >= 4096 ? 1 : 0;
-    constexpr bool okl = chain_ok<T, N, 32, LL, S::PS>() &&
-                         chain_l_lds<T, N, 32, LL, CLL>() <= kLdsBudget &&
-                         (N / 32) * LL <= 1024;
-    auto add32l = [&] {
-      if constexpr (okl) {
-        const int k = r.nchain[lg]++;
-        r.chain[lg][k] = &launch_rows_chain_l<T, N, 32, LL, S::PS, 2, CLL>;
-        r.chain_E[lg][k] = 32;
-        r.chain_lines[lg][k] = LL;
-        r.chain_twl[lg][k] = 1;
-      }
-    };
-    // 2-row tiles of 4096 points with the split compact table: two workgroups per CU
-    constexpr bool oks = N == 4096 && chain_ok<T, N, 32, S::LINES, S::PS>() &&
-                         chain_l_lds<T, N, 32, S::LINES, 2>() <= 80 * 1024;
-    auto add32s = [&] {
-      if constexpr (oks) {
-        const int k = r.nchain[lg]++;
-        r.chain[lg][k] = &launch_rows_chain_l<T, N, 32, S::LINES, S::PS, 2, 2>;
-        r.chain_E[lg][k] = 32;
-        r.chain_lines[lg][k] = S::LINES;
-        r.chain_twl[lg][k] = 1;
-      }
-    };
-    if constexpr (N == 4096) {
-      add32s();
-      add32l();
-      add32();
-      add16();
-    } else if constexpr (N >= 512) {
-      add32l();
-      add32();
-      add16();
-    } else {
-      add16();
-      add32();
-      add32l();
-    }
-    // the stack's adjoint: 16 elements per thread in row tiles of whole blocks (the
-    // group's gradient sums stay in registers beside two transforms: with 32 elements
-    // the chained form spilled 280-400 bytes per lane, and so does a 1024-thread
-    // workgroup held to 128 registers, so 2048 and 8192 keep the plane-by-plane
-    // adjoint), compact last-pass twiddles in LDS where two workgroups per CU keep
-    // room for them (at 4096 the split table with the radix-16 last pass, and the
-    // passes held to 128 registers for four waves per SIMD: 957 -> 617 us and 689 ->
-    // 519 us per 8 fields against the global tables), the global tables otherwise
-    constexpr int LA = L16;
-    constexpr int CLA = N == 4096 ? 2 : 1;
-    constexpr bool TWA = adj_chain_lds<T, N, 16, LA, CLA, true>() <= 80 * 1024;
-    if constexpr (ok16 && (N / 16) * LA <= 512 &&
-                  adj_chain_lds<T, N, 16, LA, CLA, TWA>() <= kLdsBudget) {
-      constexpr int WPA = N == 4096 ? 4 : 2;
-      r.adj_chain[lg][0] = &launch_rows_adj_chain<T, N, 16, LA, PS16, CLA, TWA, false, WPA>;
-      r.adj_chain[lg][1] = &launch_rows_adj_chain<T, N, 16, LA, PS16, CLA, TWA, true, WPA>;
-      r.adj_threads[lg] = (N / 16) * LA;
-      r.adj_lines[lg] = LA;
-    }
+  if constexpr (F32 && N == 256) {
+    add_chain<T, N, 8, 8, 0, 4>(r);
+    add_chain<T, N, 16, 16, 0, 4>(r);
+    set_adj_chain<T, N, 16, 16, 0, 4>(r);
+  } else if constexpr (F32 && N == 512) {
+    add_chain<T, N, 8, 4, 0, 4>(r);
+    add_chain<T, N, 16, 8, 4, 4>(r);
+    set_adj_chain<T, N, 16, 8, 4, 3>(r);
+  } else if constexpr (F32 && N == 1024) {
+    add_chain<T, N, 16, 4, 4, 4>(r);
+    add_chain<T, N, 32, 8, 0, 2>(r);
+    set_adj_chain<T, N, 16, 4, 4, 3>(r);
+  } else if constexpr (F32 && N == 2048) {
+    add_chain<T, N, 16, 2, 3, 4>(r);
+    add_chain<T, N, 32, 4, 4, 2>(r);
+    set_adj_chain<T, N, 16, 2, 3, 3>(r);
+  } else if constexpr (F32 && N == 4096) {
+    add_chain<T, N, 16, 2, 3, 4>(r);
+    add_chain<T, N, 32, 2, 2, 2>(r);
+    set_adj_chain<T, N, 16, 2, 3, 4>(r);
   }
   using SS = SmallShape<T, N, EMAX>;
   if constexpr (SS::OK) {

@@ -618,9 +618,13 @@ __device__ __forceinline__ void rows_body(const PassArgs<T>& a, int b, int y0, i
           dst + (size_t)(st_s * (unsigned)m) + st_o, v[m]);
 }
 
-// The row pass of one whole tile of LINES rows per workgroup.  A row's TL threads are
-// consecutive; with TL <= 64 they lie in one wave, the exchanges of the transform
-// synchronise that wave only and no wave waits for another's loads.  Few elements per
+// The row pass of one whole tile of LINES rows per workgroup.  Where a wave holds whole
+// row blocks (TiledRowMap::NAT), the exchanges of the transform synchronise that wave
+// only and no wave waits for another's loads; otherwise its barriers also keep a block
+// converted in place from being stored before every wave has loaded.  (With a row per
+// wave at TL = 64, so no barriers but half lines of the tiled plane per wave: 1024
+// points 4 fields 45.4 against 43.4 us, and the chained pass of 32 fields 146 / 126; at
+// TL = 128, 4096 points: one field 197 against 186.)  Few elements per
 // thread: many waves are resident, and they overlap their loads, arithmetic and stores
 // without a prefetch.  Bound by memory traffic: 512 fields of 256 points in 64 us each
 // way, the time of a copy of the same bytes (the persistent pass with a prefetch:
@@ -632,11 +636,13 @@ template <typename T, int N, int E, int LINES, bool INV, int PS, bool FEAT, int 
 __device__ __forceinline__ void rows_occ_body(const PassArgs<T>& a, int b, int y0, cx<T>* lds,
                                               const cx<T>* twl, int tid) {
   constexpr int TL = N / E;
-  static_assert(N % LINES == 0 && (TL > 64 || 64 % TL == 0), "whole tiles, whole waves");
-  constexpr bool WS = TL <= 64;
+  using RM = TiledRowMap<T, N, TL, LINES>;
+  static_assert(RM::ok && N % LINES == 0, "whole tiles of whole row blocks");
+  constexpr bool WS = RM::NAT;
   constexpr int L = RowPitch<N, PS, LINES>::value;
   constexpr unsigned TR = tile_rows(N);
-  const int l = tid / TL, t = tid - (tid / TL) * TL;
+  int l, t;
+  RM::map(tid, l, t);
   const int y = y0 + l;
   const bool tiled = (a.flags & F_TILED) != 0;
   const long long ubase = (long long)y0 * N;
@@ -648,7 +654,7 @@ __device__ __forceinline__ void rows_occ_body(const PassArgs<T>& a, int b, int y
   const LP2D_GLB cx<T>* __restrict__ src = field_src(a, b) + ubase;
 #pragma unroll
   for (int m = 0; m < E; ++m)
-    v[m] = gld<INV ? NT_OCCI_LD : nt_row_site<T, TL>()>(src + (size_t)(ld_s * (unsigned)m) + ld_o);
+    v[m] = gld<INV ? NT_OCCI_LD : nt_row_site<T, tiled_map_run<T, N, TL, LINES>()>()>(src + (size_t)(ld_s * (unsigned)m) + ld_o);
   if constexpr (PHO) phase_mul_all<T, E, false>(a, v, b, y, t, TL, N);
   if constexpr (FEAT) {
     if (a.flags & F_SPATIAL) {
@@ -663,12 +669,6 @@ __device__ __forceinline__ void rows_occ_body(const PassArgs<T>& a, int b, int y
   }
   LineAcc<T, PS> acc{lds + l * L};
   line_fft_l<T, N, E, INV, CL, WS>(v, t, acc, twl);
-  if constexpr (WS && (64 / TL) % (int)TR != 0) {
-    // a row block over several waves, converted in place: its other waves may still have
-    // to load (a wave's own loads are complete once it has transformed them; with
-    // TL > 64 the barriers of the transform have seen to it)
-    if (tiled) __syncthreads();
-  }
   LP2D_GLB cx<T>* __restrict__ dst = field_dst(a, b) + ubase;
   if constexpr (FEAT) {
     spatial_epi_all<T, E>(a, v, b, y, t, TL, N, (long long)b * a.fstride + (long long)y * N + t,
@@ -681,7 +681,7 @@ __device__ __forceinline__ void rows_occ_body(const PassArgs<T>& a, int b, int y
   }
 #pragma unroll
   for (int m = 0; m < E; ++m)
-    gst<INV ? nt_store_site<T>(NT_ROWI_ST, TL) : NT_ROW_ST>(dst + (size_t)(st_s * (unsigned)m) + st_o, v[m]);
+    gst<INV ? nt_store_site<T>(NT_ROWI_ST, tiled_map_run<T, N, TL, LINES>()) : NT_ROW_ST>(dst + (size_t)(st_s * (unsigned)m) + st_o, v[m]);
 }
 
 // Chained planes (a multi-plane stack u_{k+1} = P(dz)[u_k exp(i phi_k)]): the inverse
@@ -692,50 +692,49 @@ __device__ __forceinline__ void rows_occ_body(const PassArgs<T>& a, int b, int y
 // store the tile in place.  The thread map (TiledRowMap) makes every tiled access
 // cover whole tiles or 256-byte runs and every natural-order store whole 128-byte
 // lines.  Three sweeps per plane become two.
-// twl: null for the twiddles of the global table; otherwise the per-pass LDS tables of
-// twl_fill (compact last pass when CL).
-template <typename T, int N, int E, int LINES, int PS, int CL = 0>
+// Scheduled like rows_occ_body: one tile per workgroup, twiddles in LDS, the element
+// stride in the uniform base.  Bound by the plane's traffic at large batches (8 fields of
+// 4096 points with the planes stored 610 us a pass, 3.2 GB) and by latency at small ones.
+// 5 screens, forward, before (persistent, 32 elements per thread) -> now: 4 x 512^2 131 ->
+// 108 us, 1024^2 151 -> 122, 32 x 1024^2 1223 -> 1055, 8 x 2048^2 2123 -> 1432 (no chain
+// before), 8 x 4096^2 6633 -> 6329.
+template <typename T, int N, int E, int LINES, int PS, int CL>
 __device__ __forceinline__ void rows_chain_body(const PassArgs<T>& a, int b, int y0,
                                                 cx<T>* lds, const cx<T>* twl, int tid) {
   constexpr int TL = N / E;
-  constexpr int L = RowPitch<N, PS, LINES>::value;
-  constexpr int TR = tile_rows(N), TC = tile_cols<T>(N);
   using RM = TiledRowMap<T, N, TL, LINES>;
+  constexpr bool WS = RM::NAT;
+  constexpr int L = RowPitch<N, PS, LINES>::value;
+  constexpr unsigned TS = tile_rows(N) * TL;  // tiled offset step of element m
   static_assert(RM::ok && N % LINES == 0, "whole tiles of whole row blocks");
   int l, t;
   RM::map(tid, l, t);
   const int y = y0 + l;
   const long long ubase = (long long)y0 * N;
-  const unsigned lo_t = tiled_off<T, N>(l, t);
-  constexpr unsigned TS = TR * TL;  // tiled offset step of element m
+  const unsigned lo_t = tiled_off<T, N>(l, t), lo_n = (unsigned)(l * N + t);
   cx<T> v[E];
   const LP2D_GLB cx<T>* __restrict__ src = field_src(a, b) + ubase;
 #pragma unroll
-  for (int m = 0; m < E; ++m) v[m] = gld<NT_ROWI_LD>(src + (lo_t + TS * (unsigned)m));
+  for (int m = 0; m < E; ++m) v[m] = gld<NT_ROWI_LD>(src + (size_t)TS * m + lo_t);
   LineAcc<T, PS> acc{lds + l * L};
-  if (twl)
-    line_fft_l<T, N, E, true, CL>(v, t, acc, twl);
-  else
-    line_fft<T, N, E, true>(v, t, acc, a.tw_inv + (N - 2));
+  line_fft_l<T, N, E, true, CL, WS>(v, t, acc, twl);
 #pragma unroll
   for (int m = 0; m < E; ++m) v[m] = cscale(v[m], a.scale);
   if (a.flags & F_FIELD_OUT) {
     LP2D_GLB cx<T>* __restrict__ ck =
-        glb(uniform_ptr(a.field_out + (long long)b * a.fstride)) + (long long)y * N;
+        glb(uniform_ptr(a.field_out + (long long)b * a.fstride)) + ubase;
 #pragma unroll
     for (int m = 0; m < E; ++m)
-      gst<nt_store_site<T>(NT_ROWI_ST, tiled_map_run<T, N, TL, LINES>())>(ck + (t + TL * m), v[m]);
+      gst<nt_store_site<T>(NT_ROWI_ST, tiled_map_run<T, N, TL, LINES>())>(ck + (size_t)(TL * m) + lo_n, v[m]);
   }
   phase_mul_all<T, E, false>(a, v, b, y, t, TL, N);
-  if (twl)
-    line_fft_l<T, N, E, false, CL>(v, t, acc, twl);
-  else
-    line_fft<T, N, E, false>(v, t, acc, a.tw + (N - 2));
+  line_fft_l<T, N, E, false, CL, WS>(v, t, acc, twl);
   LP2D_GLB cx<T>* __restrict__ dst = field_dst(a, b) + ubase;
   // (at 4096 points with the hint: this pass 529 -> 540 us, the column pass after it
   // 765-778 -> 736 us)
 #pragma unroll
-  for (int m = 0; m < E; ++m) gst<N >= 4096 ? NT_TILE_ST : NT_ROW_ST>(dst + (lo_t + TS * (unsigned)m), v[m]);
+  for (int m = 0; m < E; ++m)
+    gst<N >= 4096 ? NT_TILE_ST : NT_ROW_ST>(dst + (size_t)TS * m + lo_t, v[m]);
 }
 
 // Adjoint of a multi-plane stack, one sweep per plane.  For the fields [b0, b1) of a
@@ -746,23 +745,25 @@ __device__ __forceinline__ void rows_chain_body(const PassArgs<T>& a, int b, int
 // order -- the gradient of the stack's input, unless F_NO_STORE -- or run the forward
 // row FFT of g and store the tile in place: the first sweep of the previous plane's
 // adjoint.  The group's sums go to `partial` (n x n) once; with partial null no
-// gradient is formed (u is not read).  Twiddles from the LDS tables twl, or from the
-// global tables when twl is null.
+// gradient is formed (u is not read).  Twiddles from the LDS tables twl.  Bound by three
+// planes of traffic (g in and out, u in): 5 screens, before -> now: 64 x 512^2 770 -> 697
+// us, 8 x 2048^2 2150 -> 1702, 8 x 4096^2 6959 -> 6787; at 4096 points the error against 64
+// bits falls from 1.2e-6 to 7.5e-7 (twiddles as one product instead of up to four).
 template <typename T, int N, int E, int LINES, int PS, int CL, bool LAST>
 __device__ __forceinline__ void rows_adj_chain_body(const PassArgs<T>& a, int b0, int b1, int y0,
                                                     float* __restrict__ partial, cx<T>* lds,
                                                     const cx<T>* twl, int tid) {
   constexpr int TL = N / E;
   constexpr int L = RowPitch<N, PS, LINES>::value;
-  constexpr int TR = tile_rows(N);
   using RM = TiledRowMap<T, N, TL, LINES>;
+  constexpr bool WS = RM::NAT;
+  constexpr unsigned TS = tile_rows(N) * TL;
   static_assert(RM::ok && N % LINES == 0, "whole tiles of whole row blocks");
   int l, t;
   RM::map(tid, l, t);
   const int y = y0 + l;
   const long long ubase = (long long)y0 * N;
-  const unsigned lo_t = tiled_off<T, N>(l, t);
-  constexpr unsigned TS = TR * TL;
+  const unsigned lo_t = tiled_off<T, N>(l, t), lo_n = (unsigned)(l * N + t);
   const bool store = (a.flags & F_NO_STORE) == 0;
   LineAcc<T, PS> acc{lds + l * L};
   float gsum[E];
@@ -776,47 +777,40 @@ __device__ __forceinline__ void rows_adj_chain_body(const PassArgs<T>& a, int b0
     cx<T> v[E];
     const LP2D_GLB cx<T>* __restrict__ src = field_src(a, b) + ubase;
 #pragma unroll
-    for (int m = 0; m < E; ++m) v[m] = gld<NT_ROWI_LD>(src + (lo_t + TS * (unsigned)m));
-    if (twl)
-      line_fft_l<T, N, E, true, CL>(v, tt, acc, twl);
-    else
-      line_fft<T, N, E, true>(v, tt, acc, a.tw_inv + (N - 2));
+    for (int m = 0; m < E; ++m) v[m] = gld<NT_ROWI_LD>(src + (size_t)TS * m + lo_t);
+    line_fft_l<T, N, E, true, CL, WS>(v, tt, acc, twl);
 #pragma unroll
     for (int m = 0; m < E; ++m) v[m] = cscale(v[m], a.scale);
     phase_mul_all<T, E, true>(a, v, b, y, tt, TL, N);
     if (partial) {
       const LP2D_GLB cx<T>* __restrict__ us =
-          glb(uniform_ptr(a.u_saved + (long long)b * a.u_sb)) + (long long)y * N;
+          glb(uniform_ptr(a.u_saved + (long long)b * a.u_sb)) + ubase;
 #pragma unroll
       for (int m = 0; m < E; ++m) {
-        const cx<T> u = gld<NT_GRAD>(us + (t + TL * m));
+        const cx<T> u = gld<NT_GRAD>(us + (size_t)(TL * m) + lo_n);
         gsum[m] += (float)(u.re * v[m].im - u.im * v[m].re);
       }
     }
     if constexpr (LAST) {
       if (store) {
-        LP2D_GLB cx<T>* __restrict__ dst = field_dst(a, b) + (long long)y * N;
+        LP2D_GLB cx<T>* __restrict__ dst = field_dst(a, b) + ubase;
 #pragma unroll
         for (int m = 0; m < E; ++m)
-          gst<nt_store_site<T>(NT_ROWI_ST, tiled_map_run<T, N, TL, LINES>())>(dst + (t + TL * m),
-                                                                          v[m]);
+          gst<nt_store_site<T>(NT_ROWI_ST, tiled_map_run<T, N, TL, LINES>())>(dst + (size_t)(TL * m) + lo_n, v[m]);
       }
     } else {
       int t2 = tt;
       asm volatile("" : "+v"(t2));
-      if (twl)
-        line_fft_l<T, N, E, false, CL>(v, t2, acc, twl);
-      else
-        line_fft<T, N, E, false>(v, t2, acc, a.tw + (N - 2));
+      line_fft_l<T, N, E, false, CL, WS>(v, t2, acc, twl);
       LP2D_GLB cx<T>* __restrict__ dst = field_dst(a, b) + ubase;
 #pragma unroll
       for (int m = 0; m < E; ++m)
-        gst<N >= 4096 ? NT_TILE_ST : NT_ROW_ST>(dst + (lo_t + TS * (unsigned)m), v[m]);
+        gst<N >= 4096 ? NT_TILE_ST : NT_ROW_ST>(dst + (size_t)TS * m + lo_t, v[m]);
     }
   }
   if (partial) {
 #pragma unroll
-    for (int m = 0; m < E; ++m) partial[(long long)y * N + t + TL * m] = gsum[m];
+    for (int m = 0; m < E; ++m) partial[ubase + (size_t)(TL * m) + lo_n] = gsum[m];
   }
 }
 

@@ -60,7 +60,6 @@ struct Registry {
   // block-tiled plane): its shapes per size (none where the plane is never tiled)
   RowChainLaunch<T> chain[kLogMax + 1][4];
   int chain_E[kLogMax + 1][4], chain_lines[kLogMax + 1][4];
-  int chain_twl[kLogMax + 1][4];  // 1: twiddles staged in LDS
   int nchain[kLogMax + 1];
   // adjoint of a stack: [0] chained (inverse rows, fold, gradient, forward rows),
   // [1] last plane (inverse rows, fold, gradient, natural store); threads per group
