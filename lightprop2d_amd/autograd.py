@@ -130,11 +130,17 @@ class StackFn(torch.autograd.Function):
                 return u
             return P.propagate_stack(u, screens_c[k0:k1], dz, area, wl)
 
-        for seg0 in reversed(range(0, K, stride)):
-            seg1 = min(K, seg0 + stride)
+        # with every plane input kept the whole stack is one segment: 2K + 1 sweeps
+        # instead of 3K (8 fields of 4096 points, 5 screens: 8.2 -> 6.8 ms)
+        kept = stride == 1 and recompute == "segment"
+        seg = K if kept else stride
+        for seg0 in reversed(range(0, K, seg)):
+            seg1 = min(K, seg0 + seg)
             ck = ctx.ckpts[seg0]
             planes = None
-            if recompute == "segment":
+            if kept:
+                planes = [ctx.ckpts[k] for k in range(K)]
+            elif recompute == "segment":
                 m = seg1 - seg0
                 planes = [ck]
                 if m > 1:  # the segment's plane inputs from one stack call
