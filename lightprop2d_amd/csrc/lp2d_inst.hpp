@@ -108,7 +108,7 @@ __global__ __launch_bounds__((N / E) * W) LP2D_OCC void k_cols(PassArgs<T> a) {
 }
 
 // Column strips by occupancy: grid (N/W strips) x (field groups of `per` fields).
-template <typename T, int N, int E, int W, int PS, int CL, bool SPEC, int WPE>
+template <typename T, int N, int E, int W, int PS, int CL, int MODE, bool MID, bool SPEC, int WPE>
 __global__ __launch_bounds__((N / E) * W) __attribute__((amdgpu_waves_per_eu(WPE)))
 void k_cols_occ(PassArgs<T> a, int per) {
   __shared__ cx<T> lds[W * PaddedLen<N, PS>::value];
@@ -120,8 +120,8 @@ void k_cols_occ(PassArgs<T> a, int per) {
   const int b0 = grp * per;
   twl_fill<T, N, E, (N / E) * W, 1, CL>(twl, a.tw, threadIdx.x);
   __syncthreads();
-  cols_occ_body<T, N, E, W, PS, CL, SPEC>(a, b0, cmin(a.batch, b0 + per), (blk - grp * SPF) * W,
-                                          lds, twl, threadIdx.x);
+  cols_occ_body<T, N, E, W, PS, CL, MODE, MID, SPEC>(
+      a, b0, cmin(a.batch, b0 + per), (blk - grp * SPF) * W, lds, twl, threadIdx.x);
 }
 
 // Whole field in LDS, pipelined over groups of `per` <= kPipeMaxPer fields.
@@ -334,15 +334,16 @@ hipError_t launch_cols_occ(const PassArgs<T>& a, int mode, hipStream_t s) {
   constexpr bool TILE_OK = (N / E) % TR == 0 && (W % TC == 0 || TC % W == 0);
   const bool ok = occ_eligible(a, mode);
   if ((a.flags & F_TILED) && (!ok || !TILE_OK)) return hipErrorInvalidValue;
+  constexpr int threads = (N / E) * W;
+  constexpr int SPF = N / W;
+  constexpr int FI = MODE_FWD | MODE_INV;
   if (ok) {
-    constexpr int threads = (N / E) * W;
-    constexpr int SPF = N / W;
     int per = 1;
     if constexpr (GMAX > 1) {
       if (a.fopt == nullptr) {
         static std::atomic<int> slot{0};
         const int slots = cached_slots(
-            slot, (const void*)&k_cols_occ<T, N, E, W, PS, CL, false, WPE>, threads);
+            slot, (const void*)&k_cols_occ<T, N, E, W, PS, CL, FI, true, false, WPE>, threads);
         int groups = slots / SPF;
         if (groups < 1) groups = 1;
         if (groups > a.batch) groups = a.batch;
@@ -352,9 +353,29 @@ hipError_t launch_cols_occ(const PassArgs<T>& a, int mode, hipStream_t s) {
     }
     const unsigned grid = (unsigned)((long long)((a.batch + per - 1) / per) * SPF);
     if (a.flags & F_SPEC_OUT)
-      k_cols_occ<T, N, E, W, PS, CL, true, WPE><<<grid, threads, 0, s>>>(a, per);
+      k_cols_occ<T, N, E, W, PS, CL, FI, true, true, WPE><<<grid, threads, 0, s>>>(a, per);
     else
-      k_cols_occ<T, N, E, W, PS, CL, false, WPE><<<grid, threads, 0, s>>>(a, per);
+      k_cols_occ<T, N, E, W, PS, CL, FI, true, false, WPE><<<grid, threads, 0, s>>>(a, per);
+    return hipGetLastError();
+  }
+  // one direction: a forward pass, or an inverse one without factor or with a transfer
+  // function (a pupil alone multiplies nothing, so infinities pass it unchanged: the plain
+  // class), one field per workgroup
+  const unsigned grid = (unsigned)((long long)a.batch * SPF);
+  const int mid = a.flags & F_MID;
+  if (mode == MODE_FWD && mid == 0) {
+    k_cols_occ<T, N, E, W, PS, CL, MODE_FWD, false, false, WPE><<<grid, threads, 0, s>>>(a, 1);
+    return hipGetLastError();
+  }
+  if (mode == MODE_INV && mid == 0) {
+    k_cols_occ<T, N, E, W, PS, CL, MODE_INV, false, false, WPE><<<grid, threads, 0, s>>>(a, 1);
+    return hipGetLastError();
+  }
+  if (mode == MODE_INV && a.evan == EV_PASS && (mid & (F_H | F_SMASK0 | F_SMASK1)) == F_H) {
+    if (mid & F_SPEC_OUT)
+      k_cols_occ<T, N, E, W, PS, CL, MODE_INV, true, true, WPE><<<grid, threads, 0, s>>>(a, 1);
+    else
+      k_cols_occ<T, N, E, W, PS, CL, MODE_INV, true, false, WPE><<<grid, threads, 0, s>>>(a, 1);
     return hipGetLastError();
   }
   return launch_cols<T, N, E, W, PS>(a, mode, s);
@@ -367,7 +388,7 @@ hipError_t launch_cols_occ(const PassArgs<T>& a, int mode, hipStream_t s) {
 template <typename T, int N, int E, int W, int PS, int CL, int GMAX, int WPE, int E2, int W2,
           int CL2, int WPE2>
 hipError_t launch_cols_pick(const PassArgs<T>& a, int mode, hipStream_t s) {
-  if (occ_eligible(a, mode) && (long long)a.batch * (N / W) < 512)
+  if ((long long)a.batch * (N / W) < 512)
     return launch_cols_occ<T, N, E2, W2, cmax(1, ilog2c(E2)), CL2, GMAX, WPE2>(a, mode, s);
   return launch_cols_occ<T, N, E, W, PS, CL, GMAX, WPE>(a, mode, s);
 }

@@ -1125,7 +1125,7 @@ __device__ __forceinline__ void pipe_stage_fields(const PassArgs<T>& a, int b0, 
   }
 }
 
-// Calls the strips by occupancy take (host side): the fused forward+inverse pass without
+// Calls the fused strips by occupancy take (host side): the forward+inverse pass without
 // mask multipliers, evanescent modes passed through.
 template <typename T>
 inline bool occ_eligible(const PassArgs<T>& a, int mode) {
@@ -1134,7 +1134,8 @@ inline bool occ_eligible(const PassArgs<T>& a, int mode) {
 }
 
 // ----------------------------------------------------------------- column strips by occupancy
-// Column FFT -> H, pupil -> column IFFT of W-column strips of fields [b0, b1), without a
+// Column FFT -> H, pupil -> column IFFT (or one of the two, MODE; MID: with the factor) of
+// W-column strips of fields [b0, b1), without a
 // prefetch: few elements per thread and short tables keep several workgroups per CU,
 // which cover one another's loads and stores.  Calls of occ_eligible.
 // The strip's factor exp(-2*pi*i*fr) x pupil is computed before the loads and held in
@@ -1151,7 +1152,7 @@ inline bool occ_eligible(const PassArgs<T>& a, int mode) {
 // Complex128, where computing the factor is the greater part of the arithmetic, this pass
 // / the plain one: 64 fields of 256 points 31 / 36 us, 16 of 512 34 / 42, 5 of 1024
 // 43 / 54, 2 of 2048 72 / 107, 1 of 4096 225 / 266.
-template <typename T, int N, int E, int W, int PS, int CL, bool SPEC>
+template <typename T, int N, int E, int W, int PS, int CL, int MODE, bool MID, bool SPEC>
 __device__ __forceinline__ void cols_occ_body(const PassArgs<T>& a, int b0, int b1, int x0,
                                               cx<T>* lds, const cx<T>* twl, int tid) {
   constexpr int TL = N / E;
@@ -1163,34 +1164,47 @@ __device__ __forceinline__ void cols_occ_body(const PassArgs<T>& a, int b0, int 
   // when tiled)
   const unsigned lo = (a.flags & F_TILED) ? tiled_off<T, N>(t, x) : lo_n;
   InterAcc<T, PS, W> acc{lds + c};
-  FieldOpt o;
-  if (a.fopt) {
-    o = a.fopt[b0];
-  } else {
-    o.k0sq = a.k0sq;
-    o.inv_ndL = a.inv_ndL;
-    o.z = a.z;
-    o.ap_r2 = a.ap_r2;
-  }
-  const ColMid cm = col_mid(o, a.flags, sx);
-  cx<T> hm[E];
+  cx<T> hm[MID ? E : 1];
+  if constexpr (MID) {
+    FieldOpt o;
+    if (a.fopt) {
+      o = a.fopt[b0];
+    } else {
+      o.k0sq = a.k0sq;
+      o.inv_ndL = a.inv_ndL;
+      o.z = a.z;
+      o.ap_r2 = a.ap_r2;
+    }
+    const ColMid cm = col_mid(o, a.flags, sx);
 #pragma unroll
-  for (int m = 0; m < E; ++m) hm[m] = mid_factor<T>(cm, t + TL * m - (m >= E / 2 ? N : 0));
+    for (int m = 0; m < E; ++m) hm[m] = mid_factor<T>(cm, t + TL * m - (m >= E / 2 ? N : 0));
+  }
   const T sc = (a.flags & F_SCALE) ? a.scale : (T)1;
   for (int b = b0; b < b1; ++b) {
     cx<T> v[E];
     const LP2D_GLB cx<T>* __restrict__ src = field_src(a, b);
 #pragma unroll
     for (int m = 0; m < E; ++m) v[m] = gld<NT_COL_LD>(src + (size_t)(TL * N) * m + lo);
-    line_fft_l<T, N, E, false, CL>(v, t, acc, twl);
+    if constexpr ((MODE & MODE_FWD) != 0) line_fft_l<T, N, E, false, CL>(v, t, acc, twl);
+    if constexpr (MID) {
 #pragma unroll
-    for (int m = 0; m < E; ++m) v[m] = cmulc(v[m], hm[m]);
+      for (int m = 0; m < E; ++m) {
+        const cx<T> r = cmulc(v[m], hm[m]);
+        if constexpr (SPEC || MODE == MODE_INV) {
+          // zero outside the pupil whatever the spectrum holds there (elsewhere |hm| = 1)
+          const bool out = hm[m].re == (T)0 && hm[m].im == (T)0;
+          v[m] = mk(out ? (T)0 : r.re, out ? (T)0 : r.im);
+        } else {
+          v[m] = r;
+        }
+      }
+    }
     if constexpr (SPEC) {
       LP2D_GLB cx<T>* __restrict__ so = glb(uniform_ptr(a.spec_out + (long long)b * a.fstride));
 #pragma unroll
       for (int m = 0; m < E; ++m) gst<NT_COL_ST>(so + (size_t)(TL * N) * m + lo_n, v[m]);
     }
-    line_fft_l<T, N, E, true, CL>(v, t, acc, twl);
+    if constexpr ((MODE & MODE_INV) != 0) line_fft_l<T, N, E, true, CL>(v, t, acc, twl);
     LP2D_GLB cx<T>* __restrict__ dst = field_dst(a, b);
 #pragma unroll
     for (int m = 0; m < E; ++m)
