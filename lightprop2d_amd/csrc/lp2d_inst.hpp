@@ -125,7 +125,7 @@ void k_cols_occ(PassArgs<T> a, int per) {
 }
 
 // Whole field in LDS, pipelined over groups of `per` <= kPipeMaxPer fields.
-template <typename T, int N, int E, int PS>
+template <typename T, int N, int E, int PS, bool PHO, bool GRAD>
 __global__ __launch_bounds__(N * (N / E)) void k_small_pipe(PassArgs<T> a, int per) {
   __shared__ cx<T> lds[N * SmallPitch<N, PS>::value];
   __shared__ cx<T> twl[TwlLen<N, E>::value];
@@ -137,7 +137,7 @@ __global__ __launch_bounds__(N * (N / E)) void k_small_pipe(PassArgs<T> a, int p
   twl_fill<T, N, E, THREADS>(twl, a.tw, threadIdx.x);
   pipe_stage_fields(a, b0, b1, pf, threadIdx.x);
   __syncthreads();
-  small_pipe_body<T, N, E, PS>(a, b0, b1, lds, twl, pf, threadIdx.x);
+  small_pipe_body<T, N, E, PS, PHO, GRAD>(a, b0, b1, lds, twl, pf, threadIdx.x);
 }
 
 template <typename T, int N, int E, int PS>
@@ -393,30 +393,41 @@ hipError_t launch_cols_pick(const PassArgs<T>& a, int mode, hipStream_t s) {
   return launch_cols_occ<T, N, E, W, PS, CL, GMAX, WPE>(a, mode, s);
 }
 
-// The fused complex64 propagation (transfer function / pupil / scale / spectrum
-// output only) runs the pipelined whole-field kernel; every other combination the
-// general one.
+// Field groups of the pipelined whole-field kernel: one resident round.
+template <typename T, int N, int E, int PS, bool PHO, bool GRAD>
+hipError_t launch_small_pipe(const PassArgs<T>& a, hipStream_t s) {
+  constexpr int threads = N * (N / E);
+  static std::atomic<int> slot{0};
+  const int slots =
+      cached_slots(slot, (const void*)&k_small_pipe<T, N, E, PS, PHO, GRAD>, threads);
+  int groups = slots < a.batch ? slots : a.batch;
+  if (groups < 1) groups = 1;
+  int per = (a.batch + groups - 1) / groups;
+  if (per > kPipeMaxPer) per = kPipeMaxPer;
+  groups = (a.batch + per - 1) / per;
+  k_small_pipe<T, N, E, PS, PHO, GRAD><<<(unsigned)groups, threads, 0, s>>>(a, per);
+  return hipGetLastError();
+}
+
+// The fused propagation (transfer function / pupil / scale / spectrum output, with or
+// without a phase screen) and its adjoint run the pipelined whole-field kernel; every
+// other combination the general one.
 template <typename T, int N, int E, int PS>
 hipError_t launch_small(const PassArgs<T>& a, int mode, hipStream_t s) {
-  constexpr int PIPE_OK_FLAGS = F_H | F_APERTURE | F_SCALE | F_SPEC_OUT;
-  if constexpr (sizeof(T) == 4 && N >= 32 && E == 16) {
-    constexpr int threads = N * (N / E);
-    constexpr int lds = N * SmallPitch<N, PS>::value * (int)sizeof(cx<T>) +
-                        TwlLen<N, E>::value * (int)sizeof(cx<T>) +
-                        kPipeMaxPer * (int)sizeof(PipeField);
-    if constexpr (lds <= kLdsBudget) {
-      if (mode == (MODE_FWD | MODE_INV) && a.evan == EV_PASS &&
-          (a.flags & ~PIPE_OK_FLAGS) == 0) {
-        static std::atomic<int> slot{0};
-        const int slots = cached_slots(slot, (const void*)&k_small_pipe<T, N, E, PS>, threads);
-        int groups = slots < a.batch ? slots : a.batch;
-        if (groups < 1) groups = 1;
-        int per = (a.batch + groups - 1) / groups;
-        if (per > kPipeMaxPer) per = kPipeMaxPer;
-        groups = (a.batch + per - 1) / per;
-        k_small_pipe<T, N, E, PS><<<(unsigned)groups, threads, 0, s>>>(a, per);
-        return hipGetLastError();
-      }
+  constexpr int BASE = F_H | F_APERTURE | F_SCALE | F_SPEC_OUT;
+  constexpr int lds = N * SmallPitch<N, PS>::value * (int)sizeof(cx<T>) +
+                      TwlLen<N, E>::value * (int)sizeof(cx<T>) +
+                      kPipeMaxPer * (int)sizeof(PipeField);
+  // (complex128 of 32 points, two waves per field: 4096 fields 39.7 us here, 34.6 in the
+  // general kernel; 64 points 74.4 -> 64.4 us for 2048 fields)
+  constexpr int NMIN = sizeof(T) == 4 ? 32 : 64;
+  if constexpr (N >= NMIN && E == (sizeof(T) == 4 ? 16 : 8) && lds <= kLdsBudget) {
+    if (mode == (MODE_FWD | MODE_INV) && a.evan == EV_PASS) {
+      const int x = a.flags & ~BASE;
+      if (x == 0) return launch_small_pipe<T, N, E, PS, false, false>(a, s);
+      if (x == F_PHASE) return launch_small_pipe<T, N, E, PS, true, false>(a, s);
+      if ((x == F_GRAD || x == (F_GRAD | F_NO_STORE)) && a.lens_rev == 0.0)
+        return launch_small_pipe<T, N, E, PS, false, true>(a, s);
     }
   }
   k_small<T, N, E, PS><<<(unsigned)a.batch, N * (N / E), 0, s>>>(a, mode);

@@ -1051,22 +1051,9 @@ __device__ __forceinline__ ColMid col_mid(const FieldOpt& o, int flags, int sx) 
   m.inv_ndL = o.inv_ndL;
   return m;
 }
-// v * H(fy) * pupil(fy) at signed frequency index sy of the column (complex64 path,
-// evanescent modes passed through).  Branch-free: same operation order as
+// The fractional phase of Kz*z and the pupil test at signed frequency index sy of the
+// column (complex64 path, evanescent modes passed through): same operation order as
 // spectral_mid for Kz^2 and the pupil test.
-__device__ __forceinline__ cx<float> mid_fast(const ColMid& m, cx<float> v, int sy) {
-#pragma clang fp contract(off)
-  const double fy = (double)sy * m.inv_ndL;
-  const double fy2 = fy * fy;
-  const float fr = kz_frac_fast(m.c0 - fy2, m.z);
-  const cx<float> h = mk(__builtin_amdgcn_cosf(fr), __builtin_amdgcn_sinf(fr));
-  const bool out = m.fx2 + fy2 > m.ap;
-  const cx<float> r = cmulc(v, h);  // exp(-2*pi*i*fr)
-  return mk(out ? 0.0f : r.re, out ? 0.0f : r.im);
-}
-
-// The FP64 part of mid_fast at signed frequency index sy: the fractional phase of
-// Kz*z and the pupil test (same operations, same order).
 __device__ __forceinline__ float mid_phase(const ColMid& m, int sy, bool& out) {
 #pragma clang fp contract(off)
   const double fy = (double)sy * m.inv_ndL;
@@ -1298,13 +1285,14 @@ __device__ __forceinline__ void small_body(const PassArgs<T>& a, int b, int mode
 // columns with H and pupil -> rows).  Twiddles and the fields' pointers and optics
 // come from LDS (twl, pf), so no wait in the loop covers the prefetch before it is
 // needed; the first field is peeled off the loop for the same reason as in the
-// column pass.  Complex64, evanescent modes passed through, no mask multipliers and
-// no spatial prologue/epilogue (flags within F_H, F_APERTURE, F_SCALE, F_SPEC_OUT).
-template <typename T, int N, int E, int PS>
+// column pass.  Evanescent modes passed through, no mask multipliers (flags within F_H,
+// F_APERTURE, F_SCALE, F_SPEC_OUT).  PHO: with a phase screen; GRAD: the adjoint's fold and
+// phase gradient (F_GRAD without a lens, F_NO_STORE).  Bound by its arithmetic: four
+// transforms and the FP64 phase, 17 us of a CU per 128-point field.
+template <typename T, int N, int E, int PS, bool PHO, bool GRAD>
 __device__ __forceinline__ void small_pipe_body(const PassArgs<T>& a, int b0, int b1,
                                                 cx<T>* lds, const cx<T>* twl,
                                                 const PipeField* pf, int tid) {
-  static_assert(sizeof(T) == 4, "complex64 path");
   constexpr int TL = N / E;
   constexpr int P = SmallPitch<N, PS>::value;
   const int flags = a.flags;
@@ -1331,6 +1319,11 @@ __device__ __forceinline__ void small_pipe_body(const PassArgs<T>& a, int b0, in
 #pragma unroll
     for (int m = 0; m < E; ++m) cur[m] = nxt[m];
     if (b + 1 < b1) fetch(b + 1);  // uniform branch
+    if constexpr (PHO) {
+      int tt = tr;  // opaque: a shared screen's factors stay out of the field loop's registers
+      asm volatile("" : "+v"(tt));
+      phase_mul_all<T, E, false>(a, cur, b, y, tt, TL, N);
+    }
     {  // rows: forward FFT into the tile
       LineAcc<T, PS> acc{lds + y * P};
       line_fft_l<T, N, E, false, 0, true>(cur, tr, acc, twl);
@@ -1350,7 +1343,12 @@ __device__ __forceinline__ void small_pipe_body(const PassArgs<T>& a, int b0, in
         int tt = tc;
         asm volatile("" : "+v"(cm.c0), "+v"(cm.fx2), "+v"(cm.inv_ndL), "+v"(tt));
 #pragma unroll
-        for (int m = 0; m < E; ++m) v[m] = mid_fast(cm, v[m], tt + TL * m - (m >= E / 2 ? N : 0));
+        for (int m = 0; m < E; ++m) {
+          const cx<T> f = mid_factor<T>(cm, tt + TL * m - (m >= E / 2 ? N : 0));
+          const cx<T> r = cmulc(v[m], f);
+          const bool out = f.re == (T)0 && f.im == (T)0;  // outside the pupil
+          v[m] = mk(out ? (T)0 : r.re, out ? (T)0 : r.im);
+        }
       }
       if (spec_out) {
         LP2D_GLB cx<T>* __restrict__ so = glb(a.spec_out + (long long)b * a.fstride + x);
@@ -1374,10 +1372,28 @@ __device__ __forceinline__ void small_pipe_body(const PassArgs<T>& a, int b0, in
 #pragma unroll
         for (int m = 0; m < E; ++m) v[m] = cscale(v[m], a.scale);
       }
-      LP2D_GLB cx<T>* __restrict__ dst =
-          glb(uniform_ptr((cx<T>*)pf[b - b0].dst)) + (long long)y * N;
+      bool store = true;
+      if constexpr (GRAD) {
+        store = (flags & F_NO_STORE) == 0;
+        int tt = tr;
+        asm volatile("" : "+v"(tt));
+        if (a.phase) phase_mul_all<T, E, true>(a, v, b, y, tt, TL, N);
+        if (a.grad_phase) {
+          const cx<T>* u = a.u_saved + (long long)b * a.u_sb + (long long)y * N + tr;
+          float* gp = a.grad_phase + (long long)b * a.fstride + (long long)y * N + tr;
 #pragma unroll
-      for (int m = 0; m < E; ++m) gst<NT_SMALL>(dst + (tr + TL * m), v[m]);
+          for (int m = 0; m < E; ++m) {
+            const cx<T> w = u[TL * m];
+            gp[TL * m] = (float)(w.re * v[m].im - w.im * v[m].re);
+          }
+        }
+      }
+      if (store) {
+        LP2D_GLB cx<T>* __restrict__ dst =
+            glb(uniform_ptr((cx<T>*)pf[b - b0].dst)) + (long long)y * N;
+#pragma unroll
+        for (int m = 0; m < E; ++m) gst<NT_SMALL>(dst + (tr + TL * m), v[m]);
+      }
     }
     __syncthreads();  // the next field's row phase rewrites the tile
   };

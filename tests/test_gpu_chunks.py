@@ -103,3 +103,37 @@ def test_stack_and_its_adjoint_match_the_planes(lib, n, K):
     assert rel_l2(gf.cpu().numpy(), x.cpu().numpy()) < tol
     for k in range(K):
         assert rel_l2(gs[k].cpu().numpy(), exp[k].cpu().numpy()) < tol, k
+
+
+@pytest.mark.parametrize("n,batch,dtype", [(32, 1, "c64"), (64, 5, "c64"), (128, 2, "c64"),
+                                           (128, 300, "c64"), (32, 3, "c128"), (64, 2, "c128"),
+                                           (64, 1100, "c128")])
+@pytest.mark.parametrize("shared", [True, False], ids=["shared", "per_field"])
+def test_whole_field_kernel_with_a_screen(n, batch, dtype, shared):
+    """One field per workgroup and several (300 and 1100 fields): forward with a phase
+    screen and a pupil, and the adjoint with its phase gradient."""
+    from lightprop2d_amd import propagation as P
+    ap = 0.4 * n / AREA
+    u, g = _field((batch, n, n), dtype, n), _field((batch, n, n), dtype, n + 1)
+    ph = torch.rand((n, n) if shared else (batch, n, n),
+                    generator=torch.Generator().manual_seed(n + batch)) * 6
+    pick = sorted({0, batch // 2, batch - 1})
+    out = P.propagate(u.to(DEV), Z, AREA, WL, phase=ph.to(DEV), aperture_radius=ap)
+    gin, gph = P.propagate_adjoint(g.to(DEV), u.to(DEV), Z, AREA, WL, phase=ph.to(DEV),
+                                   aperture_radius=ap)
+    total = np.zeros((n, n))
+    for b in range(batch) if shared else pick:
+        q = (ph if shared else ph[b]).numpy().astype(np.float64)
+        w = np.exp(-1j * q) * oracle.propagate_field(g[b].numpy(), AREA, WL, -Z,
+                                                     aperture_radius=ap)
+        grad = (np.conj(u[b].numpy().astype(np.complex128)) * w).imag
+        total += grad
+        if b in pick:
+            exp = oracle.propagate_field(u[b].numpy(), AREA, WL, Z, phase_mask=q,
+                                         aperture_radius=ap)
+            assert rel_l2(out[b].cpu().numpy(), exp) < TOL[dtype], b
+            assert rel_l2(gin[b].cpu().numpy(), w) < TOL[dtype], b
+            if not shared:
+                assert rel_l2(gph[b].cpu().numpy(), grad) < TOL["c64"], b
+    if shared:
+        assert rel_l2(gph.cpu().numpy(), total) < TOL["c64"]

@@ -84,3 +84,19 @@ def test_elementwise_sweeps_at_any_alignment(n, batch, dtype):
         assert np.abs(got - exp).max() <= 2.0 ** (-22 if dtype == "c64" else -51) * exp.max()
         P.spatial_apply(v, masks=[torch.from_numpy(mask).to(DEV)])
         assert rel_l2(v.cpu().numpy(), w * mask) < TOL_E[dtype]
+
+
+@pytest.mark.parametrize("shape,batch", [((1,), 1), ((5, 5), 3), ((17,), 4097), ((32, 32), 64),
+                                         ((33, 31), 300), ((128, 128), 65), ((512, 512), 4),
+                                         ((1024, 1024), 3)])
+def test_sum_of_planes(shape, batch):
+    """Every number of slices, odd counts, and the sum written over plane 0.  Whole numbers
+    whose sums stay below 2^24: exact in any order."""
+    from lightprop2d_amd import propagation as P
+    x = torch.randint(-1000, 1001, (batch, *shape), generator=torch.Generator().manual_seed(batch))
+    exp = x.sum(0).float()
+    x = x.float()
+    assert torch.equal(P.sum_planes(x.to(DEV), torch.empty(shape, device=DEV)).cpu(), exp)
+    buf = x.to(DEV)
+    P.sum_planes(buf, buf[0])
+    assert torch.equal(buf[0].cpu(), exp)
