@@ -987,6 +987,45 @@ int run_rows_grad(const PassArgs<T>& a, int lg, float* partial, float* out, hipS
   return LP2D_OK;
 }
 
+// Field groups of the stack adjoint's chained pass (about 512K threads in flight, no
+// empty group, as grad_groups).
+template <typename T>
+int adj_chain_groups(int lg, int batch) {
+  const Registry<T>* r = reg<T>();
+  if (!r->adj_chain[lg][0]) return 1;
+  const int tpf = (1 << lg) / r->adj_lines[lg];
+  int groups = (2048 * 256 / r->adj_threads[lg]) / tpf;
+  if (groups < 1) groups = 1;
+  if (groups > batch) groups = batch;
+  const int per = (batch + groups - 1) / groups;
+  return (batch + per - 1) / per;
+}
+
+// Inverse rows, fold of the shared screen and its gradient over the groups' planes of
+// `part` (the chained adjoint's pass `fn`), summed into `out`.
+template <typename T>
+int run_adj_chain(RowAdjChainLaunch<T> fn, const PassArgs<T>& r, int lg, int groups,
+                  const char* what, float* part, float* out, hipStream_t s) {
+  if (!out || groups == 1) part = out;
+  std::string nm;
+  if (g_trace_on) {
+    char b[64];
+    snprintf(b, sizeof(b), "rows_adj_chain n=%d %s%s", 1 << lg, tname<T>(), what);
+    nm = b;
+  }
+  hipError_t e;
+  {
+    TraceScope ts(s, nm);
+    e = fn(r, groups, part, s);
+  }
+  if (e != hipSuccess) return hip_fail(e, "adjoint chained row pass launch");
+  if (out && groups > 1) {  // (part may be out, its plane 0)
+    launch_sum_planes(part, out, 1LL << (2 * lg), groups, s);
+    if ((e = hipGetLastError()) != hipSuccess) return hip_fail(e, "sum kernel launch");
+  }
+  return LP2D_OK;
+}
+
 template <typename T>
 // scratch (allocation-free form): with a shared screen over a batch, gphase is one
 // n x n plane and the per-field or per-group gradient planes go to scratch; otherwise
@@ -1025,8 +1064,15 @@ int op_adjoint(int n, int lg, int batch, const void* gout, const void* u, const 
     a.flags = mid;
     // With a workspace the column pass writes there and the last pass reads it: no
     // in-place conversion of a tiled plane, so any gradient schedule can read one.
-    int tl = tiled_flag<T>(a, lg, shared_sum, no_store == 0 && !work);
-    const bool oop = work && tl;
+    // A shared screen's gradient takes the chained adjoint's last pass, which reads the
+    // tiled plane in whole lines at every size (8 x 2048^2 135 us against 173 in the
+    // gradient pass, 32 x 1024^2 134 / 146, 128 x 256^2 39 / 51).
+    const RowAdjChainLaunch<T> last_fn = reg<T>()->adj_chain[lg][1];
+    int tl = 0;
+    if (shared_sum && phase && last_fn) tl = tiled_flag<T>(a, lg);
+    const bool chain = tl != 0;
+    if (!chain) tl = tiled_flag<T>(a, lg, shared_sum, no_store == 0 && !work);
+    const bool oop = work && tl && !chain;
     a.flags = tl;
     if (int rc = run_rows<T>(a, lg, false, s)) return rc;
     a.src = (const cx<T>*)gin;
@@ -1036,6 +1082,12 @@ int op_adjoint(int n, int lg, int batch, const void* gout, const void* u, const 
     if (oop) {
       a.src = (const cx<T>*)work;
       a.dst = (cx<T>*)gin;
+    }
+    if (chain) {
+      a.flags = F_SCALE | no_store | tl;
+      // (no more groups than the gradient pass: the callers' workspaces are sized for it)
+      const int groups = std::min(adj_chain_groups<T>(lg, batch), grad_groups<T>(lg, batch));
+      return run_adj_chain<T>(last_fn, a, lg, groups, " last", planes, gphase, s);
     }
     if (shared_sum) {
       a.flags = F_SCALE | no_store | tl;
@@ -1051,20 +1103,6 @@ int op_adjoint(int n, int lg, int batch, const void* gout, const void* u, const 
     if (e != hipSuccess) return hip_fail(e, "sum kernel launch");
   }
   return LP2D_OK;
-}
-
-// Field groups of the stack adjoint's chained pass (about 512K threads in flight, no
-// empty group, as grad_groups).
-template <typename T>
-int adj_chain_groups(int lg, int batch) {
-  const Registry<T>* r = reg<T>();
-  if (!r->adj_chain[lg][0]) return 1;
-  const int tpf = (1 << lg) / r->adj_lines[lg];
-  int groups = (2048 * 256 / r->adj_threads[lg]) / tpf;
-  if (groups < 1) groups = 1;
-  if (groups > batch) groups = batch;
-  const int per = (batch + groups - 1) / groups;
-  return (batch + per - 1) / per;
 }
 
 // Float workspace of op_stack_adjoint: the per-group (chained pass) or per-field /
@@ -1115,7 +1153,6 @@ int op_stack_adjoint(int n, int lg, int batch, const void* gout, const void* con
     }
     return LP2D_OK;
   }
-  const int groups = adj_chain_groups<T>(lg, batch);
   a.src = (const cx<T>*)gout;
   a.dst = (cx<T>*)gin;
   a.flags = tl;
@@ -1138,24 +1175,9 @@ int op_stack_adjoint(int n, int lg, int batch, const void* gout, const void* con
     r.u_saved = gscreens ? (const cx<T>*)uk[k] : nullptr;
     r.u_sb = nn;
     r.flags = F_SCALE | tl | (k == 0 && (aflags & LP2D_ADJ_NO_GRAD_IN) ? F_NO_STORE : 0);
-    float* gk = gscreens ? gscreens + k * nn : nullptr;
-    float* part = gk && groups > 1 ? ws : gk;
-    std::string nm;
-    if (g_trace_on) {
-      char b[64];
-      snprintf(b, sizeof(b), "rows_adj_chain n=%d %s%s", n, tname<T>(), k ? "" : " last");
-      nm = b;
-    }
-    hipError_t e;
-    {
-      TraceScope ts(s, nm);
-      e = (k ? mid_fn : last_fn)(r, groups, part, s);
-    }
-    if (e != hipSuccess) return hip_fail(e, "adjoint chained row pass launch");
-    if (part && part != gk) {
-      launch_sum_planes(part, gk, nn, groups, s);
-      if ((e = hipGetLastError()) != hipSuccess) return hip_fail(e, "sum kernel launch");
-    }
+    if (int rc = run_adj_chain<T>(k ? mid_fn : last_fn, r, lg, adj_chain_groups<T>(lg, batch),
+                                  k ? "" : " last", ws, gscreens ? gscreens + k * nn : nullptr, s))
+      return rc;
   }
   return LP2D_OK;
 }

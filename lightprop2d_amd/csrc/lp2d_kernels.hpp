@@ -782,6 +782,9 @@ __device__ __forceinline__ void rows_adj_chain_body(const PassArgs<T>& a, int b0
 #pragma unroll
     for (int m = 0; m < E; ++m) v[m] = cscale(v[m], a.scale);
     phase_mul_all<T, E, true>(a, v, b, y, tt, TL, N);
+    if constexpr (LAST) {  // (a stack has no lens)
+      if (a.lens_rev != 0.0) lens_mul_all<T, E, true>(a, v, y, tt, TL, N);
+    }
     if (partial) {
       const LP2D_GLB cx<T>* __restrict__ us =
           glb(uniform_ptr(a.u_saved + (long long)b * a.u_sb)) + ubase;

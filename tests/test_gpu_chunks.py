@@ -137,3 +137,22 @@ def test_whole_field_kernel_with_a_screen(n, batch, dtype, shared):
                 assert rel_l2(gph[b].cpu().numpy(), grad) < TOL["c64"], b
     if shared:
         assert rel_l2(gph.cpu().numpy(), total) < TOL["c64"]
+
+
+@pytest.mark.parametrize("n,batch", [(256, 2), (256, 9), (512, 5), (1024, 3), (2048, 2), (4096, 2)])
+@pytest.mark.parametrize("lens", [0.0, 0.5])
+@pytest.mark.parametrize("field_grad", [True, False])
+def test_shared_screen_gradient(lib, n, batch, lens, field_grad):
+    """The adjoint of a batch under one screen, with and without a lens and the field's
+    gradient, against the per-field screens' path (which sums nothing in the pass)."""
+    from lightprop2d_amd import propagation as P
+    u, g = _field((batch, n, n), "c64", n).to(DEV), _field((batch, n, n), "c64", n + 1).to(DEV)
+    ph = torch.rand((n, n), generator=torch.Generator().manual_seed(n + batch)).to(DEV) * 6
+    gin, gph = P.propagate_adjoint(g, u, Z, AREA, WL, phase=ph, lens_f=lens,
+                                   aperture_radius=0.2 / WL, want_field_grad=field_grad)
+    per = ph.expand(batch, n, n).contiguous()
+    exp, parts = P.propagate_adjoint(g, u, Z, AREA, WL, phase=per, lens_f=lens,
+                                     aperture_radius=0.2 / WL)
+    assert rel_l2(gph.cpu().numpy(), parts.double().sum(0).cpu().numpy()) < 2 * TOL["c64"]
+    if field_grad:
+        assert rel_l2(gin.cpu().numpy(), exp.cpu().numpy()) < 2 * TOL["c64"]
