@@ -59,37 +59,39 @@ __global__ void k_coarse(const C* __restrict__ in, C* __restrict__ out, int n, i
   out[(long long)row * no + I] = o;
 }
 
-// complex64 fast paths: whole 16-byte vectors per lane.  8 fields 1024^2 <-> 2048^2:
-// expand 86.7 -> 83.5 us, coarse 70 -> 49 us (with nontemporal output stores, which
-// help the coarse mean and not the expansion).
+// complex64 fast paths: whole 16-byte vectors per lane.  8 fields 2048^2 -> 1024^2: coarse
+// 70 -> 49 us with nontemporal output stores.
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-// Expand with four output elements (i0 .. i0+3, n_out a multiple of 4) per thread,
-// written as two 16-byte stores.
-__global__ void k_expand4(const float2* __restrict__ in, float2* __restrict__ out, int n,
-                          int n_out, int d) {
+// Expand (n_out even) with kExpandPairs pairs of output elements per thread, a workgroup's
+// stores of one pair index contiguous.  Bound by the output's traffic.  8 x 1024^2 ->
+// 2048^2: 83.5 us with four neighbours per thread (two 16-byte stores 32 bytes apart between
+// lanes, each a part of its line, so no nontemporal hint), 63 with pairs, 47 with the hint
+// (335 MB); 1000 -> 1502 x 4 20.1 -> 17.
+constexpr int kExpandPairs = 2;
+__global__ __launch_bounds__(256) void k_expand2(const float2* __restrict__ in,
+                                                 float2* __restrict__ out, int n, int n_out,
+                                                 int d) {
   const int row = blockIdx.x;
   const int b = row / n_out, j = row - b * n_out;
-  const int i0 = 4 * (blockIdx.y * blockDim.x + threadIdx.x);
-  if (i0 >= n_out) return;
   int js = j - d;
   js = js < 0 ? 0 : (js >= n ? n - 1 : js);
   const float2* src = in + ((long long)b * n + js) * n;
-  float2 v[4];
+  const int t0 = 2 * (blockIdx.y * (256 * kExpandPairs) + threadIdx.x);
+  v4f v[kExpandPairs];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    int is = i0 + q - d;
-    is = is < 0 ? 0 : (is >= n ? n - 1 : is);
-    v[q] = src[is];
+  for (int q = 0; q < kExpandPairs; ++q) {
+    const int i = t0 + 512 * q;
+    int i0 = i - d, i1 = i + 1 - d;
+    i0 = i0 < 0 ? 0 : (i0 >= n ? n - 1 : i0);
+    i1 = i1 < 0 ? 0 : (i1 >= n ? n - 1 : i1);
+    const float2 a = src[i0], c = src[i1];
+    v[q].x = a.x; v[q].y = a.y; v[q].z = c.x; v[q].w = c.y;
   }
-  v4f* dst = (v4f*)(out + (long long)row * n_out + i0);
-  v4f a, c;
-  a.x = v[0].x; a.y = v[0].y; a.z = v[1].x; a.w = v[1].y;
-  c.x = v[2].x; c.y = v[2].y; c.z = v[3].x; c.w = v[3].y;
-  // plain stores: with the nontemporal hint this kernel measured 119.5 us against
-  // 83.5 us (8 x 1024^2 -> 2048^2)
-  dst[0] = a;
-  dst[1] = c;
+  v4f* dst = (v4f*)(out + (long long)row * n_out + t0);
+#pragma unroll
+  for (int q = 0; q < kExpandPairs; ++q)
+    if (t0 + 512 * q < n_out) __builtin_nontemporal_store(v[q], dst + 256 * q);
 }
 
 // 2 x 2 block mean with two outputs (I0, I0 + 1; no a multiple of 2) per thread: each
@@ -248,9 +250,10 @@ extern "C" int lp2d_expand(int n, int n_out, int batch, int dtype, const void* i
   const int d = (n_out - n) / 2;
   hipStream_t s = (hipStream_t)stream;
   const dim3 grid((unsigned)(batch * n_out), (unsigned)((n_out + 255) / 256));
-  if (dtype == LP2D_C64 && n_out % 4 == 0 && ((uintptr_t)out & 15) == 0) {
-    const dim3 g4((unsigned)(batch * n_out), (unsigned)((n_out / 4 + 255) / 256));
-    k_expand4<<<g4, 256, 0, s>>>((const float2*)in, (float2*)out, n, n_out, d);
+  if (dtype == LP2D_C64 && n_out % 2 == 0 && ((uintptr_t)out & 15) == 0) {
+    const int per = 512 * kExpandPairs;
+    const dim3 g2((unsigned)(batch * n_out), (unsigned)((n_out + per - 1) / per));
+    k_expand2<<<g2, 256, 0, s>>>((const float2*)in, (float2*)out, n, n_out, d);
   } else if (dtype == LP2D_C64)
     k_expand<float2><<<grid, 256, 0, s>>>((const float2*)in, (float2*)out, n, n_out, d);
   else

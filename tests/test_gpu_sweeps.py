@@ -100,3 +100,15 @@ def test_sum_of_planes(shape, batch):
     buf = x.to(DEV)
     P.sum_planes(buf, buf[0])
     assert torch.equal(buf[0].cpu(), exp)
+
+
+@pytest.mark.parametrize("n,n_out", [(1, 3), (2, 4), (3, 5), (4, 6), (510, 514), (512, 1026),
+                                     (500, 1024), (1000, 1502), (1024, 1024), (1024, 2050)])
+@pytest.mark.parametrize("dtype", ["c64", "c128"])
+def test_expand_is_edge_padding(n, n_out, dtype):
+    """Even and odd sizes, partial last workgroups of a row, three fields: exact copies."""
+    from lightprop2d_amd import propagation as P
+    u = _rand((3, n, n), dtype, n)
+    d = (n_out - n) // 2
+    exp = np.pad(u.numpy(), ((0, 0), (d, d), (d, d)), mode="edge")
+    assert np.array_equal(P.expand(u.to(DEV), n_out).cpu().numpy(), exp)
