@@ -1020,7 +1020,7 @@ __device__ __forceinline__ void rows_grad_pipe_body(const PassArgs<T>& a, int b0
   }
 }
 
-// ----------------------------------------------------------------- pipelined columns
+// ----------------------------------------------------------------- spectral factor
 // frac(Kz*z) in cycles for the complex64 path, with Kz = sqrt(max(kz2, 0)).  The square
 // root is v_rsq_f64 refined by one Newton step in FP64 (relative error ~1e-14, far
 // below what the FP32 phase resolves) instead of the correctly rounded expansion.
@@ -1085,7 +1085,7 @@ __device__ __forceinline__ cx<T> mid_factor(const ColMid& m, int sy) {
   }
 }
 
-// One field of a pipelined column group, staged in LDS at kernel start so that the
+// One field of a pipelined whole-field group, staged in LDS at kernel start so that the
 // field loop reads its pointers and optics without global loads (a global load there
 // would wait behind the prefetch and the previous field's stores).
 struct PipeField {
